@@ -17,6 +17,7 @@
 
 #include "../../include/lbflow.h"
 #include "device.h"
+#include "operator_f64.h"
 #include "setup.h"
 
 namespace lbf {
@@ -60,8 +61,7 @@ struct lbf_ctx {
     DevLabel* d_lab = nullptr;
     LabelF* d_lab32 = nullptr;
     DevZouHe* d_zh = nullptr;
-    double *d_AT = nullptr, *d_A = nullptr, *d_B = nullptr, *d_MInv = nullptr;
-    float *d_A32 = nullptr, *d_B32 = nullptr;
+    double *d_A4 = nullptr, *d_B4 = nullptr, *d_A = nullptr, *d_B = nullptr, *d_MInv = nullptr;
     int32_t* d_wall = nullptr;
     DevWall* d_walls = nullptr;
     WallF32* d_walls32 = nullptr;   // FP32 colour: the wall entries in FP32
@@ -134,30 +134,15 @@ double unit_component(int Q, int q, int d)
 
 int lattice_e(int Q, int q, int d) { return Q == 9 ? Lattice<9>::e[q][d] : Lattice<19>::e[q][d]; }
 
-// Pair-split form of an operator with the lattice parity symmetry (see
-// apply_split in kernels_scsp.hip).
-std::vector<float> pair_split(int Q, const std::vector<double>& op)
+// A Q x Q operator (row-major, row k = result k) in the order add_operator
+// reads it (operator_f64.h).
+std::vector<double> pack_operator(int Q, const std::vector<double>& op)
 {
-    const int H = Q == 9 ? Lattice<9>::NHALF : Lattice<19>::NHALF;
-    const int* half = Q == 9 ? Lattice<9>::half : Lattice<19>::half;
-    const int* opp = Q == 9 ? Lattice<9>::op : Lattice<19>::op;
-    std::vector<float> c(size_t((H + 1) * (H + 1) + H * H));
-    for (int r = 0; r <= H; ++r) {
-        const int q = r == 0 ? 0 : half[r - 1];
-        c[r * (H + 1)] = float(op[q * Q + 0]);
-        for (int k = 0; k < H; ++k) {
-            const int p = half[k];
-            c[r * (H + 1) + k + 1] = float(0.5 * (op[q * Q + p] + op[q * Q + opp[p]]));
-        }
-    }
-    for (int r = 1; r <= H; ++r) {
-        const int q = half[r - 1];
-        for (int k = 0; k < H; ++k) {
-            const int p = half[k];
-            c[(H + 1) * (H + 1) + (r - 1) * H + k] = float(0.5 * (op[q * Q + p] - op[q * Q + opp[p]]));
-        }
-    }
-    return c;
+    const int R = op_rows4(Q);
+    std::vector<double> out(op_packed(Q), 0.0);
+    for (int k = 0; k < Q; ++k)
+        for (int j = 0; j < Q; ++j) out[(size_t(k / 4) * R * 4 + j) * 4 + k % 4] = op[size_t(k) * Q + j];
+    return out;
 }
 
 }  // namespace
@@ -382,12 +367,11 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
         rc |= dalloc(c, &c->d_rank, (N + 31) / 32 * sizeof(uint2));
         rc |= dalloc(c, &c->d_desc_s, c->nfluid * 4);
     }
-    rc |= dalloc(c, &c->d_AT, Q2 * 8);
+    rc |= dalloc(c, &c->d_A4, op_packed(d.Q) * 8);
+    rc |= dalloc(c, &c->d_B4, op_packed(d.Q) * 8);
     rc |= dalloc(c, &c->d_A, Q2 * 8);
     rc |= dalloc(c, &c->d_B, Q2 * 8);
     rc |= dalloc(c, &c->d_MInv, Q2 * 8);
-    rc |= dalloc(c, &c->d_A32, Q2 * 4);
-    rc |= dalloc(c, &c->d_B32, Q2 * 4);
     rc |= dalloc(c, &c->d_rho0, N * 8);
     rc |= dalloc(c, &c->d_u, size_t(d.D) * N * 8);
     // adjacent history, two buffers by step parity: step t writes buffer t & 1,
@@ -451,14 +435,15 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
         }
         rc |= upload(c, c->d_zh, zh.data(), 256 * sizeof(DevZouHe));
     }
-    rc |= upload(c, c->d_AT, c->ops.AT.data(), Q2 * 8);
+    {
+        const std::vector<double> a4 = pack_operator(d.Q, c->ops.A), b4 = pack_operator(d.Q, c->ops.B);
+        rc |= upload(c, c->d_A4, a4.data(), a4.size() * 8);
+        rc |= upload(c, c->d_B4, b4.data(), b4.size() * 8);
+    }
     rc |= upload(c, c->d_A, c->ops.A.data(), Q2 * 8);
     rc |= upload(c, c->d_B, c->ops.B.data(), Q2 * 8);
     rc |= upload(c, c->d_MInv, c->ops.MInv.data(), Q2 * 8);
     {
-        std::vector<float> a32 = pair_split(d.Q, c->ops.A), b32 = pair_split(d.Q, c->ops.B);
-        rc |= upload(c, c->d_A32, a32.data(), a32.size() * 4);
-        rc |= upload(c, c->d_B32, b32.data(), b32.size() * 4);
         std::vector<LabelF> l32(256);
         for (int l = 0; l < 256; ++l) {
             std::memset(&l32[l], 0, sizeof(LabelF));
@@ -637,8 +622,8 @@ static ScspBuffers scsp_buffers(lbf_ctx* c, bool init)
     b.zh = c->d_zh;
     b.lab = c->d_lab;
     b.lab32 = c->d_lab32;
-    b.AT = c->d_AT;
-    b.B = c->d_B;
+    b.A4 = c->d_A4;
+    b.B4 = c->d_B4;
     b.rho = c->d_rho0;
     b.u = c->d_u;
     const uint64_t step = init ? 0 : c->t + 1;

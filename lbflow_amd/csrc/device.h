@@ -194,8 +194,8 @@ struct ScspBuffers {
     const uint2* rank;       // SPARSE: per 32 sites {fluid sites before them, fluid bit mask}
     const DevLabel* lab;
     const LabelF* lab32;
-    const double* AT;        // A transposed (MInvSMT of scsp.cpp:425)
-    const double* B;         // force matrix (scsp.cpp:426-427)
+    const double* A4;        // MRT collision operator (scsp.cpp:425), packed (operator_f64.h)
+    const double* B4;        // force operator (scsp.cpp:426-427), packed
     double* rho;             // fields: density
     double* u;               // fields: velocity [d][site]
     double* uadj;            // adjacent velocity history

@@ -42,6 +42,7 @@
 
 #include "collide_f32.h"
 #include "device.h"
+#include "operator_f64.h"
 #include "stream.h"
 #include "zouhe.h"
 
@@ -78,13 +79,22 @@ __device__ __forceinline__ bool resolve(const ScspParams& p, const uint32_t* __r
 
 // ---------------------------------------------------------------------------
 // FP64, reference operation order.
+//
+// Bound, MRT: half by HBM, half by FP64 issue (1444 of about 2300 FP64
+// instructions are the two operator products, add_operator).  One site per
+// lane, 151 registers, three waves per SIMD.  Measured per step on dense
+// sphere packs of porosity 0.2-0.24, before and after the operators moved from
+// LDS to scalar loads and the solid sites joined the fluid sites' loads and
+// stores: 125 x 112 x 120 229 -> 132 us (3.9 TB/s), 48^3 18.7 -> 13.4 us, an
+// SRT channel of 320 sites 6.8 -> 4.6 us; the FP32 kernel below, dense,
+// 144 x 128 x 128: 111 -> 79 us (4.6 TB/s).
 // ---------------------------------------------------------------------------
 template <int Q, bool MRT, bool INIT, int LAYOUT, bool WIDE>
 __global__ void __launch_bounds__(256)
 scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__ fout,
               const uint32_t* __restrict__ desc, const uint32_t* __restrict__ list,
               const uint2* __restrict__ rank, const DevLabel* __restrict__ lab,
-              const double* __restrict__ AT, const double* __restrict__ B, double* __restrict__ rho_out,
+              const double* __restrict__ A4, const double* __restrict__ B4, double* __restrict__ rho_out,
               double* __restrict__ u_out, double* __restrict__ uadj, DevStatus* __restrict__ status,
               const DevZouHe* __restrict__ zh)
 {
@@ -92,16 +102,6 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
     using L = Lattice<Q>;
     constexpr int D = L::D;
     using O = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
-    // The dense MRT operators are staged in LDS once per workgroup and read
-    // with uniform addresses (broadcast), before any thread leaves.
-    __shared__ double sAT[MRT ? Q * Q : 1], sB[MRT ? Q * Q : 1];
-    if constexpr (MRT) {
-        for (int k = threadIdx.x; k < Q * Q; k += 256) {
-            sAT[k] = AT[k];
-            sB[k] = B[k];
-        }
-        __syncthreads();
-    }
     uint32_t i, slot;
     if (!resolve<LAYOUT>(p, list, i, slot)) return;
     const uint32_t P = LAYOUT == SPARSE ? p.nfluid : uint32_t(p.g.N);   // plane length
@@ -109,167 +109,145 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
     const uint32_t dsc = desc[LAYOUT == SPARSE ? slot : i];
     const DevLabel* lb = lab + (dsc >> DESC_LABEL_SHIFT);
     const int kind = lb->kind;
+    const bool fluid = kind & KIND_FLUID;
+    if (!fluid && (INIT || LAYOUT != DENSE_ALL)) return;
     double f[Q];
-    Stencil stn{};
-    if (!INIT) stn = make_stencil(p.g, i);
-
-    if (!(kind & KIND_FLUID)) {
-        if (INIT || LAYOUT != DENSE_ALL) return;
-        // Solid sites are streamed but never collided, like the reference's
-        // whole-array streaming; their contents only matter for checkpoints.
-        bool finite = true;
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            f[q] = ld(fin, O(q) * P + (q == 0 ? slot : upstream<Q>(stn, q)));
-            finite = finite && isfinite(f[q]);
-            st(fout, O(q) * P + slot, f[q]);
-        }
-        if (!finite) raise_status(status, 4, p.t);
-        return;
-    }
-
-    const double force[3] = {lb->force[0], lb->force[1], D == 3 ? lb->force[2] : 0.0};
-    const bool forced = kind & KIND_FORCED;
-    if (INIT) {
-        // SCSP::initialize: f = w rho0 - 1.5 w (e.F)
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            double ef = 0.0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                if (L::e[q][d] == 1) ef += force[d];
-                else if (L::e[q][d] == -1) ef += -force[d];
-            }
-            f[q] = p.idist[q];
-            f[q] -= 1.5 * L::w[q] * ef;
-        }
-    } else {
+    if (!INIT) {
+        // Solid sites of DENSE_ALL are streamed but never collided, like the
+        // reference's whole-array streaming; their contents only matter for
+        // checkpoints.  They have no links, so their pulls and stores are the
+        // fluid sites' own instructions: a branch of their own made every
+        // mixed wave load, wait and store twice.
+        const Stencil stn = make_stencil(p.g, i);
         f[0] = ld(fin, pop_index<Q, BLK, O>(P, 0, slot));
         O off[Q];
         pull_offsets<Q, LAYOUT, O, BLK>(rank, dsc, slot, stn, p.g.nx, P, off);
 #pragma unroll
         for (int q = 1; q < Q; ++q) f[q] = ld(fin, off[q]);
     }
-
-    double rho, u[D];
-    if (kind & KIND_ZOUHE) {
-        // PB/VB: density and velocity come from the boundary, not from
-        // calcMacroVar; at t = 0 they are initialize's rho0 and 0.
+    if (fluid) {
+        const double force[3] = {lb->force[0], lb->force[1], D == 3 ? lb->force[2] : 0.0};
+        const bool forced = kind & KIND_FORCED;
         if (INIT) {
-            rho = p.dens0;
+            // SCSP::initialize: f = w rho0 - 1.5 w (e.F)
 #pragma unroll
-            for (int d = 0; d < D; ++d) u[d] = 0.0;
-        } else {
-            zouhe_f64<Q>(f, zh[dsc >> DESC_LABEL_SHIFT], rho, u);
-        }
-    } else {
-        // calcMacroVar: rho = sum_q f_q (q ascending); u = (sum +-f) / rho0
-        rho = f[0];
+            for (int q = 0; q < Q; ++q) {
+                double ef = 0.0;
 #pragma unroll
-        for (int q = 1; q < Q; ++q) rho += f[q];
-        if (!isfinite(rho) || rho <= 0.0) raise_status(status, 0, p.t);
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            double s = 0;
-#pragma unroll
-            for (int q = 1; q < Q; ++q) {
-                if (L::e[q][d] == 1) s += f[q];
-                else if (L::e[q][d] == -1) s -= f[q];
+                for (int d = 0; d < D; ++d) {
+                    if (L::e[q][d] == 1) ef += force[d];
+                    else if (L::e[q][d] == -1) ef += -force[d];
+                }
+                f[q] = p.idist[q];
+                f[q] -= 1.5 * L::w[q] * ef;
             }
-            s /= p.dens0;
-            u[d] = s;
         }
-        // bodyForce: u += (F/2)/rho0 on GV sites
-        if (kind & KIND_GV) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) u[d] += lb->half_rho[d];
-        }
-    }
-    if (p.flags & F_FIELDS) {
-        rho_out[i] = rho;
-#pragma unroll
-        for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = u[d];
-    }
-    if (p.flags & F_ADJ) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = u[d];
-    }
 
-    // collision
-    double usq = 0;
+        double rho, u[D];
+        if (kind & KIND_ZOUHE) {
+            // PB/VB: density and velocity come from the boundary, not from
+            // calcMacroVar; at t = 0 they are initialize's rho0 and 0.
+            if (INIT) {
+                rho = p.dens0;
 #pragma unroll
-    for (int d = 0; d < D; ++d) usq += u[d] * u[d];
-    if constexpr (!MRT) {
-        double uf = 0.0;
+                for (int d = 0; d < D; ++d) u[d] = 0.0;
+            } else {
+                zouhe_f64<Q>(f, zh[dsc >> DESC_LABEL_SHIFT], rho, u);
+            }
+        } else {
+            // calcMacroVar: rho = sum_q f_q (q ascending); u = (sum +-f) / rho0
+            rho = f[0];
 #pragma unroll
-        for (int d = 0; d < D; ++d) uf += u[d] * force[d];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            double ui = 0, ef = 0.0;
+            for (int q = 1; q < Q; ++q) rho += f[q];
+            if (!isfinite(rho) || rho <= 0.0) raise_status(status, 0, p.t);
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                if (L::e[q][d] == 1) { ui += u[d]; ef += force[d]; }
-                else if (L::e[q][d] == -1) { ui += -u[d]; ef += -force[d]; }
+                double s = 0;
+#pragma unroll
+                for (int q = 1; q < Q; ++q) {
+                    if (L::e[q][d] == 1) s += f[q];
+                    else if (L::e[q][d] == -1) s -= f[q];
+                }
+                if (p.dens0 != 1.0) s /= p.dens0;   // x / 1 is x
+                u[d] = s;
             }
-            const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
-            f[q] += (feq - f[q]) * p.omega;
-            // forceSource: G_q = w_q (3 (e.F - u.F) + 9 (e.u)(e.F))
-            if (forced) f[q] += p.omh * (L::w[q] * (3.0 * (ef - uf) + 9.0 * ui * ef));
-        }
-    } else {
-        double r[Q];
+            // bodyForce: u += (F/2)/rho0 on GV sites
+            if (kind & KIND_GV) {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            double ui = 0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                if (L::e[q][d] == 1) ui += u[d];
-                else if (L::e[q][d] == -1) ui += -u[d];
+                for (int d = 0; d < D; ++d) u[d] += lb->half_rho[d];
             }
-            const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
-            r[q] = feq - f[q];
         }
-        double ff[Q];
+        if (p.flags & F_FIELDS) {
+            rho_out[i] = rho;
 #pragma unroll
-        for (int qq = 0; qq < Q; ++qq) {
-            double s = 0.0;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) s += sAT[q * Q + qq] * r[q];
-            ff[qq] = s;
+            for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = u[d];
         }
+        if (p.flags & F_ADJ) {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) f[q] += ff[q];
-        if (forced) {
+            for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = u[d];
+        }
+
+        // collision
+        double usq = 0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) usq += u[d] * u[d];
+        if constexpr (!MRT) {
             double uf = 0.0;
 #pragma unroll
             for (int d = 0; d < D; ++d) uf += u[d] * force[d];
-            double src[Q];
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                double eu = 0.0, ef = 0.0;
+                double ui = 0, ef = 0.0;
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
-                    if (L::e[q][d] == 1) { eu += u[d]; ef += force[d]; }
-                    else if (L::e[q][d] == -1) { eu += -u[d]; ef += -force[d]; }
+                    if (L::e[q][d] == 1) { ui += u[d]; ef += force[d]; }
+                    else if (L::e[q][d] == -1) { ui += -u[d]; ef += -force[d]; }
                 }
-                src[q] = L::w[q] * (3.0 * (ef - uf) + 9.0 * eu * ef);
+                const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
+                f[q] += (feq - f[q]) * p.omega;
+                // forceSource: G_q = w_q (3 (e.F - u.F) + 9 (e.u)(e.F))
+                if (forced) f[q] += p.omh * (L::w[q] * (3.0 * (ef - uf) + 9.0 * ui * ef));
             }
+        } else {
+            double r[Q];
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
-                double s = 0.0;
+                double ui = 0;
 #pragma unroll
-                for (int j = 0; j < Q; ++j) s = s + src[j] * sB[q * Q + j];
-                f[q] += s;
+                for (int d = 0; d < D; ++d) {
+                    if (L::e[q][d] == 1) ui += u[d];
+                    else if (L::e[q][d] == -1) ui += -u[d];
+                }
+                const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
+                r[q] = feq - f[q];
+            }
+            add_operator<Q>(A4, r, f);
+            if (forced) {
+                double uf = 0.0;
+#pragma unroll
+                for (int d = 0; d < D; ++d) uf += u[d] * force[d];
+                double src[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    double eu = 0.0, ef = 0.0;
+#pragma unroll
+                    for (int d = 0; d < D; ++d) {
+                        if (L::e[q][d] == 1) { eu += u[d]; ef += force[d]; }
+                        else if (L::e[q][d] == -1) { eu += -u[d]; ef += -force[d]; }
+                    }
+                    src[q] = L::w[q] * (3.0 * (ef - uf) + 9.0 * eu * ef);
+                }
+                add_operator<Q>(B4, src, f);
             }
         }
     }
-    bool finite = true;
+    double chk = 0.0;   // stays 0 while every population is finite
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        finite = finite && isfinite(f[q]);
+        chk = __builtin_fma(f[q], 0.0, chk);
         st(fout, pop_index<Q, BLK, O>(P, q, slot), f[q]);
     }
-    if (!finite) raise_status(status, 4, p.t);
+    if (!(chk == 0.0)) raise_status(status, 4, p.t);
 }
 
 // ---------------------------------------------------------------------------
@@ -292,60 +270,58 @@ scsp_step_f32(ScspParams p, const float* __restrict__ fin, float* __restrict__ f
     constexpr bool BLK = LAYOUT == SPARSE;   // sparse: blocks of 64 slots
     const uint32_t dsc = desc[LAYOUT == SPARSE ? slot : i];
     const LabelF lb = lab[dsc >> DESC_LABEL_SHIFT];
+    const bool fluid = lb.kind & KIND_FLUID;
+    if (!fluid && (INIT || LAYOUT != DENSE_ALL)) return;
     float h[Q];
-    Stencil stn{};
-    if (!INIT) stn = make_stencil(p.g, i);
-
-    if (!(lb.kind & KIND_FLUID)) {
-        if (INIT || LAYOUT != DENSE_ALL) return;
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-            st(fout, O(q) * P + slot, ld(fin, O(q) * P + (q == 0 ? slot : upstream<Q>(stn, q))));
-        return;
-    }
-    const float F[3] = {lb.force[0], lb.force[1], D == 3 ? lb.force[2] : 0.0f};
-    if (INIT) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            float ef = 0.0f;
-#pragma unroll
-            for (int d = 0; d < D; ++d) ef += float(L::e[q][d]) * F[d];
-            h[q] = float(-1.5 * L::w[q]) * ef;
-        }
-    } else {
+    if (!INIT) {
+        // solid sites of DENSE_ALL: streamed with the fluid sites, not collided
+        const Stencil stn = make_stencil(p.g, i);
         h[0] = ld(fin, pop_index<Q, BLK, O>(P, 0, slot));
         O off[Q];
         pull_offsets<Q, LAYOUT, O, BLK>(rank, dsc, slot, stn, p.g.nx, P, off);
 #pragma unroll
         for (int q = 1; q < Q; ++q) h[q] = ld(fin, off[q]);
     }
-    // macro on shifted populations: rho = rho0 + sum h, j = sum e h
-    // (PB/VB: from the boundary; at t = 0 every h is 0, so drho = 0, u = 0)
-    float u[D];
-    float drho;
-    if (!INIT && (lb.kind & KIND_ZOUHE)) {
-        zouhe_f32<Q>(h, zh[dsc >> DESC_LABEL_SHIFT], p.rho0_32, drho, u);
-    } else {
-        drho = macro_f32<Q>(h, p.inv_rho0, lb.half_rho, u);
-        if (!isfinite(drho) || p.dens0 + double(drho) <= 0.0) raise_status(status, 0, p.t);
-    }
-    if (p.flags & F_FIELDS) {
-        rho_out[i] = p.dens0 + double(drho);
-#pragma unroll
-        for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = double(u[d]);
-    }
-    if (p.flags & F_ADJ) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = double(u[d]);
-    }
-    const RelaxF32 relax{p.rho0_32, p.omega32, p.omh32, p.c1_nu, p.c2_nu, p.c1_q, p.c2_q};
-    collide_f32<Q, MRT>(h, drho, u, F, relax);
     bool finite = true;
+    if (fluid) {
+        const float F[3] = {lb.force[0], lb.force[1], D == 3 ? lb.force[2] : 0.0f};
+        if (INIT) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        finite = finite && isfinite(h[q]);
-        st_pop<BLK>(fout, pop_index<Q, BLK, O>(P, q, slot), h[q]);
+            for (int q = 0; q < Q; ++q) {
+                float ef = 0.0f;
+#pragma unroll
+                for (int d = 0; d < D; ++d) ef += float(L::e[q][d]) * F[d];
+                h[q] = float(-1.5 * L::w[q]) * ef;
+            }
+        }
+        // macro on shifted populations: rho = rho0 + sum h, j = sum e h
+        // (PB/VB: from the boundary; at t = 0 every h is 0, so drho = 0, u = 0)
+        float u[D];
+        float drho;
+        if (!INIT && (lb.kind & KIND_ZOUHE)) {
+            zouhe_f32<Q>(h, zh[dsc >> DESC_LABEL_SHIFT], p.rho0_32, drho, u);
+        } else {
+            drho = macro_f32<Q>(h, p.inv_rho0, lb.half_rho, u);
+            if (!isfinite(drho) || p.dens0 + double(drho) <= 0.0) raise_status(status, 0, p.t);
+        }
+        if (p.flags & F_FIELDS) {
+            rho_out[i] = p.dens0 + double(drho);
+#pragma unroll
+            for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = double(u[d]);
+        }
+        if (p.flags & F_ADJ) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = double(u[d]);
+        }
+        const RelaxF32 relax{p.rho0_32, p.omega32, p.omh32, p.c1_nu, p.c2_nu, p.c1_q, p.c2_q};
+        collide_f32<Q, MRT>(h, drho, u, F, relax);
+        float chk = 0.0f;   // stays 0 while every population is finite
+#pragma unroll
+        for (int q = 0; q < Q; ++q) chk = fmaf(h[q], 0.0f, chk);
+        finite = chk == 0.0f;
     }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) st_pop<BLK>(fout, pop_index<Q, BLK, O>(P, q, slot), h[q]);
     if (!finite) raise_status(status, 4, p.t);
 }
 
@@ -365,7 +341,7 @@ static void launch_scsp_w(const ScspParams& p, const ScspBuffers& b, bool fp32, 
     else
         hipLaunchKernelGGL((scsp_step_f64<Q, MRT, INIT, LAYOUT, WIDE>), grid, block, 0, s, p,
                            static_cast<const double*>(b.fin), static_cast<double*>(b.fout), b.desc, b.list,
-                           b.rank, b.lab, b.AT, b.B, b.rho, b.u, b.uadj, b.status, b.zh);
+                           b.rank, b.lab, b.A4, b.B4, b.rho, b.u, b.uadj, b.status, b.zh);
 }
 
 template <int Q, bool MRT, bool INIT, int LAYOUT>

@@ -103,7 +103,6 @@ void build_mrt(int Q, double tau, MrtOperators& out)
     std::vector<double> h(Q);
     for (int k = 0; k < Q; ++k) h[k] = 1.0 - 0.5 * out.S[k];
     out.A = matmul(scale_columns(out.MInv, out.S.data(), Q), out.M, Q, Q, Q);
-    out.AT = transpose(out.A, Q, Q);
     out.B = matmul(scale_columns(out.MInv, h.data(), Q), out.M, Q, Q, Q);
 }
 

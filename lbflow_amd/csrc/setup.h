@@ -20,7 +20,7 @@ struct LabelInfo {
 // (solver/src/lbm/simulator.cpp:162-216, scsp.cpp:420-427, colorfluid.cpp:315-322).
 struct MrtOperators {
     int Q = 0;
-    std::vector<double> M, MInv, S, A, AT, B;   // row-major Q*Q (S: Q)
+    std::vector<double> M, MInv, S, A, B;   // row-major Q*Q (S: Q)
 };
 void build_mrt(int Q, double tau, MrtOperators& out);
 // Relaxation rates S(tau) of Simulator::getMRTS (legacy spectrum).

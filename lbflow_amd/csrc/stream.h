@@ -62,15 +62,12 @@ __device__ __forceinline__ O pull_offset(const uint2* __restrict__ rank, uint32_
                                          const Stencil& st, uint32_t P, int q)
 {
     using L = Lattice<Q>;
-    // site x - e_q solid <=> site in ibS[op(q)] (simulator.cpp:103-111)
-    if ((links >> L::op[q]) & 1u) return O(L::op[q]) * P + slot;
-    const uint32_t src = upstream<Q>(st, q);
-    if constexpr (LAYOUT == SPARSE) {
-        const uint2 r = rank[src >> 5];
-        return O(q) * P + (r.x + uint32_t(__popc(r.y & ((1u << (src & 31u)) - 1u))));
-    } else {
-        return O(q) * P + src;
-    }
+    static_assert(LAYOUT != SPARSE, "the sparse layout looks up whole rows (pull_offsets)");
+    // site x - e_q solid <=> site in ibS[op(q)] (simulator.cpp:103-111); both
+    // offsets are formed and one selected: a branch per direction cost more
+    // instructions than the two additions it skipped, and split the loads
+    const O back = O(L::op[q]) * P + slot, pull = O(q) * P + upstream<Q>(st, q);
+    return ((links >> L::op[q]) & 1u) ? back : pull;
 }
 
 // Element index of plane q of slot s in an array of NPL planes.  The dense
