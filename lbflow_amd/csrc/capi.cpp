@@ -55,13 +55,17 @@ struct lbf_ctx {
     uint64_t pop_elems = 0;         // elements of one population buffer
     size_t elem = 8;
     uint32_t* d_desc = nullptr;
+    // FP64 colour: the step's work order and the fluid sites alone (setup.h build_items)
+    uint2 *d_items = nullptr, *d_fitems = nullptr;
+    uint32_t nitems = 0, nfitems = 0;
+    bool plain = false;             // no label of the geometry is PB, VB or HF
     uint32_t* d_list = nullptr;
     uint2* d_rank = nullptr;         // sparse: per 32 sites {fluid sites before, fluid mask}
     uint32_t* d_desc_s = nullptr;    // sparse: descriptor per slot
     DevLabel* d_lab = nullptr;
     LabelF* d_lab32 = nullptr;
     DevZouHe* d_zh = nullptr;
-    double *d_A4 = nullptr, *d_B4 = nullptr, *d_A = nullptr, *d_B = nullptr, *d_MInv = nullptr;
+    double *d_A4 = nullptr, *d_B4 = nullptr, *d_MI4 = nullptr;
     int32_t* d_wall = nullptr;
     DevWall* d_walls = nullptr;
     WallF32* d_walls32 = nullptr;   // FP32 colour: the wall entries in FP32
@@ -95,6 +99,10 @@ int fail(lbf_ctx* c, const std::string& msg)
     else g_create_error = msg;
     return -1;
 }
+
+// Waves per region of a work order (setup.h build_items): 1024 entries, four
+// workgroups.
+constexpr uint32_t REGION_WAVES = 16;
 
 #define HIP_CHECK(ctx, expr)                                                                   \
     do {                                                                                       \
@@ -211,11 +219,13 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
     }
     // Labels used by the geometry must be supported by the kernels.
     {
+        c->plain = true;
         bool used[256] = {false};
         for (uint64_t i = 0; i < N; ++i) used[geometry[i]] = true;
         for (int l = 0; l < 256; ++l) {
             if (!used[l] || !labels[l].type) continue;
             const int t = labels[l].type;
+            if (t == LBF_PB || t == LBF_VB || t == LBF_HF) c->plain = false;
             if (t == LBF_AB) {
                 lbf_destroy(c);
                 return fail(nullptr, "lbf_create: label " + std::to_string(l) +
@@ -354,7 +364,6 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
     }
     (void)hipGetDevice(&c->device);
     const size_t pop = c->pop_elems * c->elem;
-    const size_t Q2 = size_t(d.Q) * d.Q;
     int rc = 0;
     rc |= dalloc(c, &c->f[0], pop);
     rc |= dalloc(c, &c->f[1], pop);
@@ -362,6 +371,22 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
     rc |= dalloc(c, &c->d_lab, 256 * sizeof(DevLabel));
     rc |= dalloc(c, &c->d_lab32, 256 * sizeof(LabelF));
     rc |= dalloc(c, &c->d_zh, 256 * sizeof(DevZouHe));
+    std::vector<SiteItem> items, fitems;
+    if (NP == 2 && c->elem == 8) {
+        bool fluid_label[256];
+        for (int l = 0; l < 256; ++l) fluid_label[l] = c->hlab[l].kind & KIND_FLUID;
+        if (d.flags & LBF_STREAM_SOLIDS)
+            build_items(N, c->links.desc.data(), fluid_label, true, REGION_WAVES, items);
+        build_items(N, c->links.desc.data(), fluid_label, false, REGION_WAVES, fitems);
+        if (items.size() >= ITEM_NONE) {
+            lbf_destroy(c);
+            return fail(nullptr, "lbf_create: lattice too large for 32-bit site indices");
+        }
+        c->nitems = uint32_t(items.size());
+        c->nfitems = uint32_t(fitems.size());
+        rc |= dalloc(c, &c->d_items, items.size() * sizeof(SiteItem));
+        rc |= dalloc(c, &c->d_fitems, fitems.size() * sizeof(SiteItem));
+    }
     if (c->layout == 2) {
         rc |= dalloc(c, &c->d_list, c->nfluid * 4);
         rc |= dalloc(c, &c->d_rank, (N + 31) / 32 * sizeof(uint2));
@@ -369,9 +394,7 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
     }
     rc |= dalloc(c, &c->d_A4, op_packed(d.Q) * 8);
     rc |= dalloc(c, &c->d_B4, op_packed(d.Q) * 8);
-    rc |= dalloc(c, &c->d_A, Q2 * 8);
-    rc |= dalloc(c, &c->d_B, Q2 * 8);
-    rc |= dalloc(c, &c->d_MInv, Q2 * 8);
+    rc |= dalloc(c, &c->d_MI4, op_packed(d.Q) * 8);
     rc |= dalloc(c, &c->d_rho0, N * 8);
     rc |= dalloc(c, &c->d_u, size_t(d.D) * N * 8);
     // adjacent history, two buffers by step parity: step t writes buffer t & 1,
@@ -409,6 +432,8 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
         return fail(nullptr, e);
     }
     rc |= upload(c, c->d_desc, c->links.desc.data(), N * 4);
+    if (c->d_items) rc |= upload(c, c->d_items, items.data(), items.size() * sizeof(SiteItem));
+    if (c->d_fitems) rc |= upload(c, c->d_fitems, fitems.data(), fitems.size() * sizeof(SiteItem));
     rc |= upload(c, c->d_lab, c->hlab.data(), 256 * sizeof(DevLabel));
     {
         // Zou-He boundaries (scsp.cpp:188-256); FP32 constants as in DevZouHe
@@ -436,13 +461,12 @@ int lbf_create(const lbf_desc* desc, const lbf_label* labels, const uint8_t* geo
         rc |= upload(c, c->d_zh, zh.data(), 256 * sizeof(DevZouHe));
     }
     {
-        const std::vector<double> a4 = pack_operator(d.Q, c->ops.A), b4 = pack_operator(d.Q, c->ops.B);
+        const std::vector<double> a4 = pack_operator(d.Q, c->ops.A), b4 = pack_operator(d.Q, c->ops.B),
+                                  m4 = pack_operator(d.Q, c->ops.MInv);
+        rc |= upload(c, c->d_MI4, m4.data(), m4.size() * 8);
         rc |= upload(c, c->d_A4, a4.data(), a4.size() * 8);
         rc |= upload(c, c->d_B4, b4.data(), b4.size() * 8);
     }
-    rc |= upload(c, c->d_A, c->ops.A.data(), Q2 * 8);
-    rc |= upload(c, c->d_B, c->ops.B.data(), Q2 * 8);
-    rc |= upload(c, c->d_MInv, c->ops.MInv.data(), Q2 * 8);
     {
         std::vector<LabelF> l32(256);
         for (int l = 0; l < 256; ++l) {
@@ -637,6 +661,11 @@ static ColorArgs color_args(lbf_ctx* c, uint32_t flags)
     ColorArgs a{};
     a.g = c->g;
     a.desc = c->d_desc;
+    a.items = c->d_items;
+    a.nitems = c->nitems;
+    a.fitems = c->d_fitems;
+    a.nfitems = c->nfitems;
+    a.plain = c->plain && uint64_t(2) * c->Q * c->N * 8 < (uint64_t(1) << 32);
     a.lab = c->d_lab;
     a.wall = c->d_wall;
     a.walls = c->d_walls;
@@ -650,9 +679,9 @@ static ColorArgs color_args(lbf_ctx* c, uint32_t flags)
     a.sigma = c->d.sigma;
     a.renormalized = c->d.wall_gradient == LBF_WALL_RENORMALIZED;
     a.densN = c->d_densN;
-    a.A = c->d_A;
-    a.B = c->d_B;
-    a.MInv = c->d_MInv;
+    a.A4 = c->d_A4;
+    a.B4 = c->d_B4;
+    a.MI4 = c->d_MI4;
     a.rho0 = c->d_rho0;
     a.rho1 = c->d_rho1;
     a.u = c->d_u;

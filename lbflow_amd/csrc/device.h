@@ -207,14 +207,20 @@ struct ColorArgs {
     GridDev g;
     const double* fin;       // [phase][q][site]
     double* fout;
+    // FP64: work orders {site, descriptor} (setup.h build_items) of the step
+    // that streams solids and of the passes that only visit fluid sites
+    const uint2 *items, *fitems;
+    uint32_t nitems, nfitems;
     const uint32_t* desc;
     const DevLabel* lab;
     const int32_t* wall;
     const DevWall* walls;
     double* densN;           // colour indicator with solid sentinel
-    const double* A;         // uniform-tau collision matrix (row-major)
-    const double* B;         // uniform-tau force matrix
-    const double* MInv;      // inverse transform (row-major)
+    // FP64 operators packed for add_operator (operator_f64.h): the uniform-tau
+    // collision and force matrices and the inverse transform
+    const double *A4, *B4, *MI4;
+    // FP64: no PB, VB or HF site, and both population sets below 4 GiB
+    int32_t plain;
     double* rho0;
     double* rho1;
     double* u;

@@ -26,7 +26,21 @@
 //
 // FP64, reference operation order (built with -ffp-contract=off); zero
 // lattice coefficients are skipped exactly as in kernels_scsp.hip.
+//
+// Bound: FP64 issue and, on lattices of a few waves per SIMD, the step's own
+// chain of cold loads and cold code (220 registers, two waves per SIMD).
+// Waves hold either fluid or solid sites (setup.h build_items), the operators
+// come through scalar loads (operator_f64.h; through vector loads they were 480
+// round trips), directions are divided by the gradient's norm once per opposite
+// pair (65 -> 36 divisions), and lattices without PB, VB or HF sites run a
+// kernel without those branches.  Measured per step, before and after: rock of
+// 48^3 (porosity 0.24) 49.7 -> 34.8 us, 96^3 425 -> 253 us, 256 x 128 x 128
+// (porosity 0.3) 2062 -> 1232 us, a 2D channel of 544 sites 13.9 -> 9.3 us.
+#include <type_traits>
+
 #include "device.h"
+#include "operator_f64.h"
+#include "stream.h"
 #include "zouhe.h"
 
 namespace lbf {
@@ -36,15 +50,29 @@ constexpr double SQRT2 = 1.4142135623730951;  // sqrt(2.0), Qnorm of diagonal li
 
 namespace {
 
+// This thread's entry of a work order.
+__device__ __forceinline__ bool resolve_color(const uint2* __restrict__ items, uint32_t n, uint32_t& site,
+                                              uint32_t& desc)
+{
+    const uint32_t k = xcd_block() * 256u + threadIdx.x;
+    if (k >= n) return false;
+    const uint2 it = items[k];
+    site = it.x;
+    desc = it.y;
+    return it.x != ITEM_NONE;
+}
+
 // Pull (or initialise) both phases; returns the total fT_q = f0_q + f1_q and
 // the phase densities summed in direction order.  PB/VB sites apply the
 // Zou-He boundary to the pulled populations first and return its density and
 // velocity in rzh / uzh.  OWN (with INIT): the site's own populations in fin,
 // not streamed (the capillary initialisation's second macro pass).
-template <int Q, bool INIT, bool OWN = false>
+// PLAIN: the lattice has no PB, VB or HF site and both population sets lie
+// below 4 GiB (32-bit byte offsets).
+template <int Q, bool INIT, bool OWN, bool PLAIN>
 __device__ __forceinline__ void load_color(const ColorArgs& a, uint32_t i, uint32_t desc,
-                                           const DevLabel& lab, double* fT, double& r0, double& r1,
-                                           double& rzh, double* uzh)
+                                           const DevLabel& lab, const Stencil& stn, double* fT, double& r0,
+                                           double& r1, double& rzh, double* uzh)
 {
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
@@ -75,10 +103,8 @@ __device__ __forceinline__ void load_color(const ColorArgs& a, uint32_t i, uint3
         }
         return;
     }
-    int x, y, z;
-    site_coords(a.g, i, x, y, z);
     const uint32_t links = desc & DESC_LINK_MASK;
-    if ((lab.kind & (KIND_ZOUHE | KIND_FILM)) || (desc & DESC_FILM)) {
+    if (!PLAIN && ((lab.kind & (KIND_ZOUHE | KIND_FILM)) || (desc & DESC_FILM))) {
         // Boundary sites, in the reference's order: bounce-back at solid
         // links, then each phase bounces back at links into a film of the
         // other phase, the film empties the other phase (clearHalfFilm,
@@ -91,7 +117,7 @@ __device__ __forceinline__ void load_color(const ColorArgs& a, uint32_t i, uint3
             int qs = q;
             if (q == 0) src = i;
             else if ((links >> L::op[q]) & 1u) { src = i; qs = L::op[q]; }
-            else src = pull_source<Q>(a.g, x, y, z, q);
+            else src = upstream<Q>(stn, q);
             const bool back0 = q != 0 && ((film >> L::op[q]) & 1u);
             const bool back1 = q != 0 && ((film >> (32 + L::op[q])) & 1u);
             f0[q] = a.fin[uint64_t(back0 ? L::op[q] : qs) * N + (back0 ? i : src)];
@@ -113,44 +139,57 @@ __device__ __forceinline__ void load_color(const ColorArgs& a, uint32_t i, uint3
         }
         return;
     }
+    using O = typename std::conditional<PLAIN, uint32_t, uint64_t>::type;
+    const O P = O(N), plane1 = O(Q) * P;
+    O off[Q];
+    off[0] = i;
+    pull_offsets<Q, DENSE_ALL, O>(nullptr, links, i, stn, a.g.nx, uint32_t(N), off);
+    double f1[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        uint64_t src;
-        int qs = q;
-        if (q == 0) src = i;
-        else if ((links >> L::op[q]) & 1u) { src = i; qs = L::op[q]; }
-        else src = pull_source<Q>(a.g, x, y, z, q);
-        const double f0 = a.fin[uint64_t(qs) * N + src];
-        const double f1 = a.fin[(uint64_t(Q) + qs) * N + src];
-        if (q == 0) { r0 = f0; r1 = f1; }
-        else { r0 += f0; r1 += f1; }
-        fT[q] = f0 + f1;
+        fT[q] = ld(a.fin, off[q]);
+        f1[q] = ld(a.fin, off[q] + plane1);
     }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        if (q == 0) { r0 = fT[q]; r1 = f1[q]; }
+        else { r0 += fT[q]; r1 += f1[q]; }
+        fT[q] = fT[q] + f1[q];
+    }
+}
+
+// The colour indicator at the site (dn[0]) and at x + e_q (dn[q], the pull
+// source of the opposite direction).
+template <int Q>
+__device__ __forceinline__ void gather_indicator(const ColorArgs& a, uint32_t i, const Stencil& stn, double* dn)
+{
+    using L = Lattice<Q>;
+    dn[0] = a.densN[i];
+#pragma unroll
+    for (int q = 1; q < Q; ++q) dn[q] = a.densN[upstream<Q>(stn, L::op[q])];
 }
 
 // Colour gradient of a fluid site from the rhoN stencil (ColorFluid::
 // colorGradient, colorfluid.cpp:435-570): bulk stencil, or at wall sites the
 // one-sided stencil over fluid neighbours, the renormalized or tanh
 // reconstruction, and the geometric contact-angle rotation.  Returns |g|.
+// w is the site's wall entry, dn its indicator stencil (gather_indicator).
 template <int Q>
-__device__ __forceinline__ double color_gradient_f64(const ColorArgs& a, uint32_t i, int x, int y, int z,
-                                                     double* g)
+__device__ __forceinline__ double color_gradient_f64(const ColorArgs& a, int32_t w, const double* dn, double* g)
 {
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
     constexpr int D = L::D;
     g[0] = g[1] = g[2] = 0.0;
     double norm;
-    const int32_t w = a.wall[i];
     if (!w) {
 #pragma unroll
         for (int d = 0; d < D; ++d)
 #pragma unroll
             for (int k = 0; k < L::NREL; ++k) {
                 const int q = L::reld[d][k];
-                const double dnq = a.densN[push_target<Q>(a.g, x, y, z, q)];
-                if (L::e[q][d] == 1) g[d] += L::w[q] * dnq;
-                else g[d] -= L::w[q] * dnq;
+                if (L::e[q][d] == 1) g[d] += L::w[q] * dn[q];
+                else g[d] -= L::w[q] * dn[q];
             }
 #pragma unroll
         for (int d = 0; d < D; ++d) g[d] *= 3.0;
@@ -159,16 +198,17 @@ __device__ __forceinline__ double color_gradient_f64(const ColorArgs& a, uint32_
         for (int d = 0; d < D; ++d) n2 = n2 + g[d] * g[d];
         norm = sqrt(n2);
     } else {
-        const double dn0 = a.densN[i];
+        // a solid neighbour adds nothing: + 0 leaves a sum as it is
+        double step[Q];
+#pragma unroll
+        for (int q = 1; q < Q; ++q) step[q] = dn[q] == SOLID_DENS_N ? 0.0 : L::w[q] * (dn[q] - dn[0]);
 #pragma unroll
         for (int d = 0; d < D; ++d)
 #pragma unroll
             for (int k = 0; k < L::NREL; ++k) {
                 const int q = L::reld[d][k];
-                const double dnq = a.densN[push_target<Q>(a.g, x, y, z, q)];
-                if (dnq == SOLID_DENS_N) continue;
-                if (L::e[q][d] == 1) g[d] += L::w[q] * (dnq - dn0);
-                else g[d] -= L::w[q] * (dnq - dn0);
+                if (L::e[q][d] == 1) g[d] += step[q];
+                else g[d] -= step[q];
             }
 #pragma unroll
         for (int d = 0; d < D; ++d) g[d] *= 3.0;
@@ -267,7 +307,7 @@ __device__ __forceinline__ double color_gradient_f64(const ColorArgs& a, uint32_
 // with d_b c_a from the inverse moment at wall sites, else 3 sum w e dc;
 // F = sigma/2 kappa direction.  Returns false if F is not finite.
 template <int Q>
-__device__ __forceinline__ bool capillary_force(const ColorArgs& a, uint32_t i, int x, int y, int z, double* F)
+__device__ __forceinline__ bool capillary_force(const ColorArgs& a, uint32_t i, const Stencil& stn, double* F)
 {
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
@@ -288,7 +328,7 @@ __device__ __forceinline__ bool capillary_force(const ColorArgs& a, uint32_t i, 
         bool fluid[Q];
 #pragma unroll
         for (int q = 1; q < Q; ++q) {
-            nb[q] = push_target<Q>(a.g, x, y, z, q);
+            nb[q] = upstream<Q>(stn, L::op[q]);
             fluid[q] = a.densN[nb[q]] != SOLID_DENS_N;
         }
 #pragma unroll
@@ -338,17 +378,15 @@ __device__ __forceinline__ bool capillary_force(const ColorArgs& a, uint32_t i, 
 
 }  // namespace
 
-template <int Q, bool INIT, bool OWN = false>
+template <int Q, bool INIT, bool OWN = false, bool PLAIN = false>
 __global__ void __launch_bounds__(256) color_density(ColorArgs a)
 {
 #pragma clang fp contract(off)
-    const uint32_t i = xcd_block() * 256u + threadIdx.x;
-    if (i >= a.g.N) return;
-    const uint32_t desc = a.desc[i];
+    uint32_t i, desc;
+    if (!resolve_color(a.fitems, a.nfitems, i, desc)) return;
     const DevLabel& lab = a.lab[desc >> DESC_LABEL_SHIFT];
-    if (!(lab.kind & KIND_FLUID)) return;
     double fT[Q], r0, r1, rzh, uzh[Lattice<Q>::D];
-    load_color<Q, INIT, OWN>(a, i, desc, lab, fT, r0, r1, rzh, uzh);
+    load_color<Q, INIT, OWN, PLAIN>(a, i, desc, lab, make_stencil(a.g, i), fT, r0, r1, rzh, uzh);
     const double rt = r0 + r1;
     a.densN[i] = (r0 - r1) / rt;
 }
@@ -361,15 +399,12 @@ __global__ void __launch_bounds__(256) color_capillary(ColorArgs a)
 {
 #pragma clang fp contract(off)
     constexpr int D = Lattice<Q>::D;
-    const uint32_t i = xcd_block() * 256u + threadIdx.x;
-    if (i >= a.g.N) return;
+    uint32_t i, desc;
+    if (!resolve_color(a.fitems, a.nfitems, i, desc)) return;
     const uint64_t N = a.g.N;
-    const uint32_t desc = a.desc[i];
-    if (!(a.lab[desc >> DESC_LABEL_SHIFT].kind & KIND_FLUID)) return;
-    int x, y, z;
-    site_coords(a.g, i, x, y, z);
-    double g[3];
-    const double norm = color_gradient_f64<Q>(a, i, x, y, z, g);
+    double g[3], dn[Q];
+    gather_indicator<Q>(a, i, make_stencil(a.g, i), dn);
+    const double norm = color_gradient_f64<Q>(a, a.wall[i], dn, g);
 #pragma unroll
     for (int d = 0; d < D; ++d) {
         a.capgrad[uint64_t(d) * N + i] = g[d];
@@ -388,12 +423,11 @@ __global__ void __launch_bounds__(256) color_tanh_wall(ColorArgs a)
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
     constexpr int D = L::D;
-    const uint32_t i = xcd_block() * 256u + threadIdx.x;
-    if (i >= a.g.N) return;
+    uint32_t i, desc;
+    if (!resolve_color(a.fitems, a.nfitems, i, desc)) return;
     const int32_t w = a.wall[i];
-    if (!w || !(a.lab[a.desc[i] >> DESC_LABEL_SHIFT].kind & KIND_FLUID)) return;
-    int x, y, z;
-    site_coords(a.g, i, x, y, z);
+    if (!w) return;
+    const Stencil stn = make_stencil(a.g, i);
     const DevWall& wl = a.walls[w];
     const double dn0 = a.densN[i];
     double g[3];
@@ -401,7 +435,7 @@ __global__ void __launch_bounds__(256) color_tanh_wall(ColorArgs a)
     double moment[3] = {0.0, 0.0, 0.0}, slope[3];
 #pragma unroll
     for (int q = 1; q < Q; ++q) {
-        const double nb = a.densN[push_target<Q>(a.g, x, y, z, q)];
+        const double nb = a.densN[upstream<Q>(stn, L::op[q])];
         if (nb == SOLID_DENS_N) continue;
         const double difference = tanh_wall_transform(nb) - center;
 #pragma unroll
@@ -448,12 +482,10 @@ __global__ void __launch_bounds__(256) color_csf_init(ColorArgs a)
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
     constexpr int D = L::D;
-    const uint32_t i = xcd_block() * 256u + threadIdx.x;
-    if (i >= a.g.N) return;
+    uint32_t i, desc;
+    if (!resolve_color(a.fitems, a.nfitems, i, desc)) return;
     const uint64_t N = a.g.N;
-    const uint32_t desc = a.desc[i];
     const DevLabel& lab = a.lab[desc >> DESC_LABEL_SHIFT];
-    if (!(lab.kind & KIND_FLUID)) return;
     const int ph = lab.phase;
     const double* dist = ph == 0 ? a.dist0 : a.dist1;
     double f0[Q], f1[Q], r0, r1;
@@ -467,10 +499,8 @@ __global__ void __launch_bounds__(256) color_csf_init(ColorArgs a)
         else { r0 += f0[q]; r1 += f1[q]; }
     }
     const double rt = r0 + r1;
-    int x, y, z;
-    site_coords(a.g, i, x, y, z);
     double F[3] = {0.0, 0.0, 0.0};
-    if (!capillary_force<Q>(a, i, x, y, z, F)) raise_status(a.status, 5, a.t);
+    if (!capillary_force<Q>(a, i, make_stencil(a.g, i), F)) raise_status(a.status, 5, a.t);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         double ef = 0.0;
@@ -486,51 +516,63 @@ __global__ void __launch_bounds__(256) color_csf_init(ColorArgs a)
     }
 }
 
-template <int Q, bool MRT, bool INIT, bool STREAM_SOLIDS, bool CSF = false, bool OWN = false>
+template <int Q, bool MRT, bool INIT, bool STREAM_SOLIDS, bool CSF = false, bool OWN = false, bool PLAIN = false>
 __global__ void __launch_bounds__(256) color_step(ColorArgs a)
 {
 #pragma clang fp contract(off)
     using L = Lattice<Q>;
     constexpr int D = L::D;
-    const uint32_t i = xcd_block() * 256u + threadIdx.x;
-    if (i >= a.g.N) return;
+    uint32_t i, desc;
+    if (!resolve_color(STREAM_SOLIDS ? a.items : a.fitems, STREAM_SOLIDS ? a.nitems : a.nfitems, i, desc)) return;
     const uint64_t N = a.g.N;
-    const uint32_t desc = a.desc[i];
     const DevLabel& lab = a.lab[desc >> DESC_LABEL_SHIFT];
     const int kind = lab.kind;
 
-    if (!(kind & KIND_FLUID)) {
-        if (INIT || !STREAM_SOLIDS) return;
-        int x, y, z;
-        site_coords(a.g, i, x, y, z);
-        bool finite = true;
+    using O = typename std::conditional<PLAIN, uint32_t, uint64_t>::type;
+    const O P = O(N);
+    const Stencil stn = make_stencil(a.g, i);
+    if (STREAM_SOLIDS && !(desc & ITEM_FLUID)) {
+        double f0[Q], f1[Q], chk = 0.0;
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
-            const uint64_t src = q == 0 ? i : pull_source<Q>(a.g, x, y, z, q);
-            const double f0 = a.fin[uint64_t(q) * N + src];
-            const double f1 = a.fin[(uint64_t(Q) + q) * N + src];
-            finite = finite && isfinite(f0) && isfinite(f1);
-            a.fout[uint64_t(q) * N + i] = f0;
-            a.fout[(uint64_t(Q) + q) * N + i] = f1;
+            const O src = q == 0 ? i : upstream<Q>(stn, q);
+            f0[q] = ld(a.fin, O(q) * P + src);
+            f1[q] = ld(a.fin, O(Q + q) * P + src);
         }
-        if (!finite) raise_status(a.status, 4, a.t);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            chk = __builtin_fma(f0[q], 0.0, __builtin_fma(f1[q], 0.0, chk));
+            st(a.fout, O(q) * P + O(i), f0[q]);
+            st(a.fout, O(Q + q) * P + O(i), f1[q]);
+        }
+        if (!(chk == 0.0)) raise_status(a.status, 4, a.t);
         return;
     }
 
+    // The indicator stencil and the wall entry are requested with the
+    // populations, and the colour gradient is formed first: it frees the
+    // stencil before the collision needs the registers.
+    double dn[Q], g[3] = {0.0, 0.0, 0.0}, norm = 0.0;
+    int32_t wall = 0;
+    if constexpr (!CSF) {
+        wall = a.wall[i];
+        gather_indicator<Q>(a, i, stn, dn);
+    }
     double fT[Q], r0, r1, rzh = 0.0, uzh[D];
-    load_color<Q, INIT, OWN>(a, i, desc, lab, fT, r0, r1, rzh, uzh);
+    load_color<Q, INIT, OWN, PLAIN>(a, i, desc, lab, stn, fT, r0, r1, rzh, uzh);
+    if constexpr (!CSF) norm = color_gradient_f64<Q>(a, wall, dn, g);
 
-    // calcMacroVar
+    // calcMacroVar (a sum of two is finite only if both are)
     const double rt = r0 + r1;
-    if (!isfinite(r0) || !isfinite(r1) || !isfinite(rt) || rt <= 0.0) raise_status(a.status, 0, a.t);
+    if (!(rt > 0.0) || rt == HUGE_VAL) raise_status(a.status, 0, a.t);
     else if (r0 < -1e-10 * rt || r1 < -1e-10 * rt) raise_status(a.status, 1, a.t);
-    const double dn = (r0 - r1) / rt;
-    double tau = (1 + dn) * a.relax0 + (1 - dn) * a.relax1;
+    const double chi = (r0 - r1) / rt;
+    double tau = (1 + chi) * a.relax0 + (1 - chi) * a.relax1;
     if (a.harmonic) {
         const double phi = r0 / rt;
         tau = 0.5 + 3.0 / (phi / a.nu0 + (1.0 - phi) / a.nu1);
     }
-    if (!isfinite(tau) || tau <= 0.5) raise_status(a.status, 2, a.t);
+    if (!(tau > 0.5) || tau == HUGE_VAL) raise_status(a.status, 2, a.t);
     double u[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -542,21 +584,25 @@ __global__ void __launch_bounds__(256) color_step(ColorArgs a)
         }
         s /= rt;
         u[d] = s;
-        if (!isfinite(s)) raise_status(a.status, 3, a.t);
+    }
+    {
+        double chk = 0.0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) chk = __builtin_fma(u[d], 0.0, chk);
+        if (!(chk == 0.0)) raise_status(a.status, 3, a.t);
     }
     // bodyForce (colorfluid.cpp:736-750): under CSF first u += (F_cap/2)/rho
     // on VD/GV sites, then u += (F/2)/rho on GV sites
     double fcap[3] = {0.0, 0.0, 0.0};
     if constexpr (CSF) {
-        int cx, cy, cz;
-        site_coords(a.g, i, cx, cy, cz);
-        if (!capillary_force<Q>(a, i, cx, cy, cz, fcap)) raise_status(a.status, 5, a.t);
+        if (!capillary_force<Q>(a, i, stn, fcap)) raise_status(a.status, 5, a.t);
 #pragma unroll
         for (int d = 0; d < D; ++d) u[d] += .5 * fcap[d] / rt;
     }
     if (kind & KIND_GV) {
 #pragma unroll
-        for (int d = 0; d < D; ++d) u[d] += lab.half[d] / rt;
+        for (int d = 0; d < D; ++d)
+            if (lab.half[d] != 0.0) u[d] += lab.half[d] / rt;   // the force has few components
     }
     if (a.flags & 1u) {
         a.rho0[i] = r0;
@@ -654,24 +700,8 @@ __global__ void __launch_bounds__(256) color_step(ColorArgs a)
         }
         double corr[Q];
         if (a.uniform) {
-            const double* __restrict__ A = a.A;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double s = 0.0;
-#pragma unroll
-                for (int j = 0; j < Q; ++j) s = s + res[j] * A[q * Q + j];
-                corr[q] = s;
-            }
-            if (forced) {
-                const double* __restrict__ B = a.B;
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    double s = 0.0;
-#pragma unroll
-                    for (int j = 0; j < Q; ++j) s = s + src[j] * B[q * Q + j];
-                    corr[q] += s;
-                }
-            }
+            add_operator<Q, true>(a.A4, res, corr);
+            if (forced) add_operator<Q>(a.B4, src, corr);
         } else {
             // per-site rates S(tau) in moment space (colorfluid.cpp:379-383)
             const double su = 1.0 / tau;
@@ -705,26 +735,14 @@ __global__ void __launch_bounds__(256) color_step(ColorArgs a)
                     m[k] += g * (1.0 - 0.5 * rate);
                 }
             }
-            const double* __restrict__ MI = a.MInv;
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double s = 0.0;
-#pragma unroll
-                for (int k = 0; k < Q; ++k)
-                    if (L::M[k][q] != 0) s = s + m[k] * MI[q * Q + k];
-                corr[q] = s;
-            }
+            add_operator<Q, true, true>(a.MI4, m, corr);
         }
 #pragma unroll
         for (int q = 0; q < Q; ++q) fT[q] += corr[q];
     }
 
     // colour gradient: the stored capillary gradient under CSF (no
-    // perturbation, colorfluid.cpp:389-411), else colorGradient
-    int x, y, z;
-    site_coords(a.g, i, x, y, z);
-    double g[3] = {0.0, 0.0, 0.0};
-    double norm;
+    // perturbation, colorfluid.cpp:389-411), else colorGradient above
     if constexpr (CSF) {
         double n2 = 0.0;
 #pragma unroll
@@ -733,18 +751,28 @@ __global__ void __launch_bounds__(256) color_step(ColorArgs a)
             n2 = n2 + g[d] * g[d];
         }
         norm = sqrt(n2);
-    } else {
-        norm = color_gradient_f64<Q>(a, i, x, y, z, g);
     }
 
-    // perturbation + recolouring
+    // perturbation + recolouring.  e_q . g / norm only changes its sign
+    // between opposite directions, and so do the products built on it: one
+    // division (two on the diagonals) serves a pair.
     const double dens0T = r0 / rt;
-    bool finite = true;
-    if (norm > 1e-9) {
+    double chk = 0.0;   // f1 = fT - f0 is finite only if both are
+    const bool interface = norm > 1e-9;
+    auto put = [&](int q, double f0) __attribute__((always_inline)) {
+        const double f1 = fT[q] - f0;
+        chk = __builtin_fma(f1, 0.0, chk);
+        st(a.fout, O(q) * P + O(i), f0);
+        st(a.fout, O(Q + q) * P + O(i), f1);
+    };
+    if (interface) {
         const double b01 = a.beta * dens0T * r1 / rt;
         const double akn = a.ak * norm / tau;
+        if constexpr (!CSF) fT[0] += akn * (0.0 - a.bi[0]);
+        put(0, dens0T * fT[0]);
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
+        for (int j = 0; j < L::NHALF; ++j) {
+            const int q = L::half[j], o = L::op[q];
             double angle = 0.0;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
@@ -752,44 +780,45 @@ __global__ void __launch_bounds__(256) color_step(ColorArgs a)
                 else if (L::e[q][d] == -1) angle -= g[d];
             }
             angle /= norm;
-            if constexpr (!CSF) fT[q] += akn * (L::w[q] * angle * angle - a.bi[q]);
+            if constexpr (!CSF) {
+                const double bend = L::w[q] * angle * angle;
+                fT[q] += akn * (bend - a.bi[q]);
+                fT[o] += akn * (bend - a.bi[o]);
+            }
             if (L::diagonal(q)) angle /= SQRT2;
-            const double f0 = dens0T * fT[q] + b01 * angle * feq0[q];
-            const double f1 = fT[q] - f0;
-            finite = finite && isfinite(f0) && isfinite(f1);
-            a.fout[uint64_t(q) * N + i] = f0;
-            a.fout[(uint64_t(Q) + q) * N + i] = f1;
+            const double turn = b01 * angle;
+            put(q, dens0T * fT[q] + turn * feq0[q]);
+            put(o, dens0T * fT[o] - turn * feq0[o]);
         }
     } else {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const double f0 = dens0T * fT[q];
-            const double f1 = fT[q] - f0;
-            finite = finite && isfinite(f0) && isfinite(f1);
-            a.fout[uint64_t(q) * N + i] = f0;
-            a.fout[(uint64_t(Q) + q) * N + i] = f1;
-        }
+        for (int q = 0; q < Q; ++q) put(q, dens0T * fT[q]);
     }
-    if (!finite) raise_status(a.status, 4, a.t);
+    if (!(chk == 0.0)) raise_status(a.status, 4, a.t);
 }
 
 template <int Q, bool MRT, bool INIT>
 static hipError_t launch_color_q(const ColorArgs& a, bool stream_solids, hipStream_t s)
 {
-    const dim3 grid(uint32_t((a.g.N + 255) / 256)), block(256);
+    // passes over the fluid sites, and the step's own order
+    const dim3 grid((a.nfitems + 255) / 256), all((a.nitems + 255) / 256), block(256);
+    const bool fluid = a.nfitems != 0;
+    if (!fluid && (INIT || !stream_solids)) return hipSuccess;
     auto tanh_pass = [&](const ColorArgs& x) {
-        if (x.tanh_wall) hipLaunchKernelGGL((color_tanh_wall<Q>), grid, block, 0, s, x);
+        if (x.tanh_wall && fluid) hipLaunchKernelGGL((color_tanh_wall<Q>), grid, block, 0, s, x);
     };
     if (a.csf) {
         // CSF (colorfluid.cpp:124-137): a step is density, gradient/curvature
         // field, step.  t = 0: initialize + calcMacroVar, the capillary shift
         // of the populations, calcMacroVar again, bodyForce and collision on
         // the shifted populations in place.
-        hipLaunchKernelGGL((color_density<Q, INIT>), grid, block, 0, s, a);
-        tanh_pass(a);
-        hipLaunchKernelGGL((color_capillary<Q>), grid, block, 0, s, a);
+        if (fluid) {
+            hipLaunchKernelGGL((color_density<Q, INIT>), grid, block, 0, s, a);
+            tanh_pass(a);
+            hipLaunchKernelGGL((color_capillary<Q>), grid, block, 0, s, a);
+        }
         if (!INIT) {
-            if (stream_solids) hipLaunchKernelGGL((color_step<Q, MRT, false, true, true>), grid, block, 0, s, a);
+            if (stream_solids) hipLaunchKernelGGL((color_step<Q, MRT, false, true, true>), all, block, 0, s, a);
             else hipLaunchKernelGGL((color_step<Q, MRT, false, false, true>), grid, block, 0, s, a);
             return hipGetLastError();
         }
@@ -802,9 +831,19 @@ static hipError_t launch_color_q(const ColorArgs& a, bool stream_solids, hipStre
         hipLaunchKernelGGL((color_step<Q, MRT, true, false, true, true>), grid, block, 0, s, b);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL((color_density<Q, INIT>), grid, block, 0, s, a);
+    if constexpr (!INIT)
+        if (a.plain) {
+            if (fluid) hipLaunchKernelGGL((color_density<Q, false, false, true>), grid, block, 0, s, a);
+            tanh_pass(a);
+            if (stream_solids)
+                hipLaunchKernelGGL((color_step<Q, MRT, false, true, false, false, true>), all, block, 0, s, a);
+            else
+                hipLaunchKernelGGL((color_step<Q, MRT, false, false, false, false, true>), grid, block, 0, s, a);
+            return hipGetLastError();
+        }
+    if (fluid) hipLaunchKernelGGL((color_density<Q, INIT>), grid, block, 0, s, a);
     tanh_pass(a);
-    if (stream_solids && !INIT) hipLaunchKernelGGL((color_step<Q, MRT, INIT, true>), grid, block, 0, s, a);
+    if (stream_solids && !INIT) hipLaunchKernelGGL((color_step<Q, MRT, INIT, true>), all, block, 0, s, a);
     else hipLaunchKernelGGL((color_step<Q, MRT, INIT, false>), grid, block, 0, s, a);
     return hipGetLastError();
 }

@@ -120,5 +120,9 @@ constexpr unsigned DESC_LINK_MASK = 0x7ffffu;
 // Bit 19: the site has a link into a half-permeable film site of the other
 // phase for one of its phases (the per-site film word holds which).
 constexpr unsigned DESC_FILM = 1u << 19;
+// Bit 20, in the work order of the dense layouts only: a fluid site.
+constexpr unsigned ITEM_FLUID = 1u << 20;
+// Work-order entry that pads a wave.
+constexpr unsigned ITEM_NONE = 0xffffffffu;
 
 }  // namespace lbf

@@ -262,6 +262,30 @@ std::string wall_gradient_inverse(int D, int Q, const uint64_t* sz, const LabelI
     return "";
 }
 
+void build_items(uint64_t N, const uint32_t* desc, const bool* fluid_label, bool solids, uint32_t region_waves,
+                 std::vector<SiteItem>& out)
+{
+    constexpr uint64_t WAVE = 64;
+    std::vector<SiteItem> fluid, solid;
+    out.clear();
+    auto flush = [&]() {
+        for (std::vector<SiteItem>* v : {&fluid, &solid}) {
+            out.insert(out.end(), v->begin(), v->end());
+            while (out.size() % WAVE) out.push_back(SiteItem{ITEM_NONE, 0u});
+            v->clear();
+        }
+    };
+    for (uint64_t i = 0; i < N; ++i) {
+        const bool f = fluid_label[desc[i] >> DESC_LABEL_SHIFT];
+        if (!f && !solids) continue;
+        std::vector<SiteItem>& v = f ? fluid : solid;
+        const uint64_t waves = (fluid.size() + WAVE - 1) / WAVE + (solid.size() + WAVE - 1) / WAVE;
+        if (waves == region_waves && v.size() % WAVE == 0) flush();   // this site would open a wave too many
+        v.push_back(SiteItem{uint32_t(i), desc[i] | (f ? ITEM_FLUID : 0u)});
+    }
+    flush();
+}
+
 FastDiv make_fastdiv(uint32_t d)
 {
     FastDiv f;

@@ -50,6 +50,22 @@ std::string wall_gradient_inverse(int D, int Q, const uint64_t* sz, const LabelI
 std::string build_links(int D, int Q, const uint64_t* sz, const LabelInfo* labels,
                         const uint8_t* geometry, bool rotations, Links& out);
 
+// Work order of a kernel that visits the sites of a dense layout: every site
+// once as {site, descriptor}, in waves of 64 entries that hold either fluid
+// sites (ITEM_FLUID set in the descriptor) or solid ones, the last wave of
+// each run padded with ITEM_NONE.  A fluid wave costs a collision, a solid
+// one only the copy of its populations; 64 consecutive sites of a rock nearly
+// always hold both and pay for a collision with a quarter of their lanes.
+// Sites are taken in regions of as many consecutive sites as fill
+// region_waves waves, fluid waves first, so the lines that both kinds touch
+// are read and written by a few neighbouring workgroups of one XCD.
+// solids = false leaves solid sites out.
+struct SiteItem {
+    uint32_t site, desc;
+};
+void build_items(uint64_t N, const uint32_t* desc, const bool* fluid_label, bool solids, uint32_t region_waves,
+                 std::vector<SiteItem>& out);
+
 // Periodic neighbour of site i along lattice vector e (components slowest first).
 uint64_t neighbour(int D, const uint64_t* sz, uint64_t i, const int* e);
 
