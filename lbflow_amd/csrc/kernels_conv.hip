@@ -13,7 +13,7 @@
 // channels-last activations and k = tap * Cin + ci, one lane's 8 k are 8
 // consecutive channels of one voxel: a single 16-byte load.
 //
-// Forward: a workgroup of 4 waves covers 256 voxels x BN output channels;
+// Forward (direct kernel): a workgroup of 4 waves covers 256 voxels x BN output channels;
 // each wave owns 64 voxels (4 row tiles) x BN.  A is loaded straight from
 // memory into MFMA registers (neighbour gather, 16 B per lane); the weight
 // panel is staged through LDS (128 k per stage, rows padded by 32 B: 72
@@ -366,6 +366,208 @@ conv_fwd_halo(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restric
                 obase[i][r * os + 16 * j] = OutT(x);
             }
     }
+}
+
+// ---------------------------------------------------------------------------
+// forward (and input gradient), 3x3x3 with Cin a multiple of 32, BF16 output,
+// sides >= 16.
+//
+// A wave computes XT x RY tiles of 16 consecutive x voxels (XT tiles along x,
+// RY rows along y, one z layer) times BN output channels; the 4 waves of a
+// workgroup stack along z.  Per 32-channel chunk the workgroup's input with its
+// one-voxel periodic halo lies in LDS (64 bytes per voxel).  The taps run in
+// order; for one dz the fragments of a wave's RY + 2 input rows at the 3 x
+// shifts are read once each and serve all taps dy: 36 LDS reads instead of 72
+// for the 144 products of XT RY = 8, BN = 32.
+//
+// Two workgroups share a CU, so that one copies its tile (straight from memory
+// into LDS) or stores while the other computes.  A wave of 8 row tiles reads
+// 2 KB of weights per 16 products; with 4 row tiles and 64 output channels the
+// weight stream filled the L1 (192 to 64 channels 337 us, so 202 us).  Also
+// measured: one workgroup per CU with two LDS tiles, copying the next step's
+// tile during the products, took longer (145-186 us against 123 us, 32 to 32
+// channels): loads return in order, and the weights queue behind the copies.
+//
+// The activations are the B operand and the weights the A operand: a lane's
+// results are then output channels of one voxel, and with the weight rows
+// permuted between a pair of tiles they are 8 consecutive channels, one
+// 16-byte store (2-byte stores with the operands the other way round).
+//
+// LDS voxel v holds the 8-channel group c at chunk c ^ ((v >> 1) & 3): the 16
+// lanes of a group read 16 consecutive voxels without bank conflicts (measured
+// against strides of 64, 80 and 96 bytes and four other swizzles).  A row is 2
+// (mod 8) voxels long, so a lane needs 4 addresses per x shift and every read
+// is one of them plus a constant.
+// ---------------------------------------------------------------------------
+template <int XT, int RY> struct RowsShape {
+    static constexpr int BX = 16 * XT, BY = RY, BZ = 4, VOX = BX * BY * BZ;
+    static constexpr int HX = BX + 2, HY = BY + 2, HZ = BZ + 2, HV = HX * HY * HZ;
+    static constexpr int COPIES = (HV + 63) / 64;              // copy instructions of a copying wave per tile
+    static constexpr int TILE = (HV + 15) / 16 * 16 * 32;      // BF16 of one LDS tile
+};
+
+template <int CIN, int COUT, int BN, int XT, int RY, int ACT, bool BIAS>
+__global__ void __launch_bounds__(256, 2)
+conv_fwd_rows(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restrict__ w,
+              const float* __restrict__ bias, __bf16* __restrict__ out)
+{
+    using H = RowsShape<XT, RY>;
+    constexpr int KP = conv_kp(CIN, 27), NT = BN / 16, T = XT * RY, CC = 32, NB = COUT / BN;
+    constexpr int AHEAD = 3, RING = AHEAD + 1;                 // taps of weights in flight
+    static_assert(CIN % CC == 0 && BN % 32 == 0 && COUT % BN == 0 && H::HX % 8 == 2, "shape");
+    static_assert(64 / H::HX + 1 < H::HY, "one carry per copy");
+    __shared__ __attribute__((aligned(16))) __bf16 tile[H::TILE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, grp = lane >> 4;
+    const uint32_t ls = g.log_s, S = 1u << ls, m = S - 1u;
+    // workgroup -> output channels (the blocks of channels of one block of
+    // voxels follow each other on one XCD), sample, block origin
+    const uint32_t bps = (1u << (3 * ls)) / H::VOX, nbx = S / H::BX, nby = S / H::BY;
+    const uint32_t wg = xcd_block(), blk = wg / NB, smp = blk / bps, b = blk % bps;
+    const int co0 = int(wg % NB) * BN;
+    const uint32_t x0 = (b % nbx) * H::BX, y0 = ((b / nbx) % nby) * H::BY, z0 = (b / (nbx * nby)) * H::BZ;
+    const size_t sbase = size_t(smp) << (3 * ls);
+
+    // LDS byte addresses of the lane's voxel at x shift dx, one per row mod 4
+    const uint32_t lds0 = uint32_t(uintptr_t((__attribute__((address_space(3))) __bf16*)tile));
+    uint32_t at[3][4];
+#pragma unroll
+    for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t v = uint32_t(wave * H::HY * H::HX + dx + r16);
+            at[dx][k] = lds0 + v * 64u + ((uint32_t(grp) ^ (((v >> 1) + uint32_t(k)) & 3u)) << 4);
+        }
+    // weight rows of a pair of tiles: result 4 a + r of tile 2 p + q is output channel 32 p + 8 a + 4 q + r
+    uint32_t wrow[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+        wrow[j] = uint32_t(co0 + 32 * (j / 2) + 8 * (r16 >> 2) + 4 * (j & 1) + (r16 & 3)) * KP + 8 * grp;
+    // halo coordinates of the first voxel this lane copies
+    const uint32_t sv = uint32_t(16 * wave + (lane >> 2)), srow = sv / uint32_t(H::HX);
+    const uint32_t sx = sv - srow * H::HX, sz = srow / uint32_t(H::HY), sy = srow - sz * H::HY;
+    f32x4 acc[T][NT];
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    // split over input channels (gridDim.y > 1): this workgroup's chunks
+    const int cps = (CIN / CC) / int(gridDim.y);
+    const int c_begin = int(blockIdx.y) * cps * CC, c_end = c_begin + cps * CC;
+#pragma unroll 1
+    for (int c0 = c_begin; c0 < c_end; c0 += CC) {
+        if (c0 != c_begin) __syncthreads();   // the previous chunk's reads are done with the tile
+        // 16 voxels per instruction, lane l fills chunk l % 4 of voxel l / 4.
+        // The wave's next 16 voxels are 64 further on, reached with carries.
+        const char* src = reinterpret_cast<const char*>(in + sbase * g.in_stride + c0);
+        uint32_t hx = sx, hy = sy, hz = sz;
+#pragma unroll 4
+        for (int n = 0; n < H::COPIES; ++n) {
+            const uint32_t v = uint32_t(64 * n) + sv;
+            const uint32_t x = (x0 + hx - 1u) & m, y = (y0 + hy - 1u) & m, z = (z0 + hz - 1u) & m;
+            const uint32_t c = (uint32_t(lane) & 3u) ^ ((v >> 1) & 3u);
+            const uint32_t off = ((z << (2 * ls)) | (y << ls) | x) * (2u * g.in_stride) + 16u * c;
+            if (v < uint32_t(H::HV))
+                __builtin_amdgcn_global_load_lds(
+                    (const __attribute__((address_space(1))) void*)(src + off),
+                    (__attribute__((address_space(3))) void*)(tile + (64 * n + 16 * wave) * CC), 16, 0, 0);
+            hx += 64 % H::HX;
+            hy += 64 / H::HX;
+            const bool cx = hx >= uint32_t(H::HX);
+            hx -= cx ? H::HX : 0;
+            hy += cx ? 1 : 0;
+            const bool cy = hy >= uint32_t(H::HY);
+            hy -= cy ? H::HY : 0;
+            hz += cy ? 1 : 0;
+        }
+        const __bf16* wc = w + c0;
+        bf16x8 wf[RING][NT], a[RY + 2][XT][3];
+        auto weights = [&](int tap) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                wf[tap % RING][j] = *reinterpret_cast<const bf16x8*>(wc + tap * CIN + wrow[j]);
+        };
+        auto rows = [&](int dz, int first, int last, int dx) __attribute__((always_inline)) {
+            typedef const __attribute__((address_space(3))) bf16x8 lbf;
+#pragma unroll
+            for (int r = first; r <= last; ++r)
+#pragma unroll
+                for (int h = 0; h < XT; ++h) {
+                    const int row = dz * H::HY + r;
+                    a[r][h][dx] = *(lbf*)(uintptr_t(at[dx][row & 3]) + uint32_t((row * H::HX + 16 * h) * 64));
+                }
+        };
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t) weights(t);
+        // this wave's copies into LDS have landed; the barrier then covers the others'
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        // What a tap needs is requested two or three taps before it: the weights
+        // AHEAD taps before, a further input row with the taps of the previous
+        // dy, the next dz's first rows for shift dx once the last tap that
+        // reads the old ones has been issued.  The scheduling barriers keep
+        // the requests there; left alone they move down to their uses, and a
+        // wave then waits out each of them.
+        rows(0, 0, RY - 1, 0);
+        rows(0, 0, RY - 1, 1);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int tap = 0; tap < 27; ++tap) {
+            const int dz = tap / 9, dy = tap / 3 % 3, dx = tap % 3;
+            if (tap + AHEAD < 27) weights(tap + AHEAD);
+            if (dy < 2) rows(dz, RY + dy, RY + dy, dx);
+            if (dy == 0 && dx == 0) rows(dz, 0, RY - 1, 2);
+            if (dy == 2 && dx && dz < 2) rows(dz + 1, 0, RY - 1, dx - 1);
+#pragma unroll
+            for (int y = 0; y < RY; ++y)
+#pragma unroll
+                for (int h = 0; h < XT; ++h)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j)
+                        acc[y * XT + h][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            wf[tap % RING][j], a[dy + y][h][dx], acc[y * XT + h][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    // a lane holds, per tile and pair of channel tiles, 8 consecutive channels of one voxel
+    const uint32_t ch = uint32_t(co0 + 8 * grp);
+    float bs[NT / 2][8];
+    if constexpr (BIAS)
+#pragma unroll
+        for (int p = 0; p < NT / 2; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) bs[p][e] = bias[ch + 32 * p + e];
+#pragma unroll
+    for (int y = 0; y < RY; ++y)
+#pragma unroll
+        for (int h = 0; h < XT; ++h) {
+            const size_t v = sbase + ((size_t(z0 + wave) << (2 * ls)) | (size_t(y0 + y) << ls) | (x0 + 16 * h + r16));
+#pragma unroll
+            for (int p = 0; p < NT / 2; ++p) {
+                const f32x4 lo = acc[y * XT + h][2 * p], hi = acc[y * XT + h][2 * p + 1];
+                const uint32_t co = ch + 32 * p;
+                if (gridDim.y > 1) {
+                    // split: this split's FP32 partial, summed by conv_ksplit_sum
+                    float* kb = g.kpart + (size_t(blockIdx.y) * g.nvox + v) * COUT + co;
+                    *reinterpret_cast<f32x4*>(kb) = lo;
+                    *reinterpret_cast<f32x4*>(kb + 4) = hi;
+                    continue;
+                }
+                bf16x8 gate, o;
+                if constexpr (ACT == ACT_RELU_GATE)
+                    gate = *reinterpret_cast<const bf16x8*>(g.gate + v * g.gate_stride + co);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    float r = e < 4 ? lo[e & 3] : hi[e & 3];
+                    if constexpr (BIAS) r += bs[p][e];
+                    if (ACT == ACT_RELU) r = r > 0.0f ? r : 0.0f;
+                    if constexpr (ACT == ACT_RELU_GATE) r = float(gate[e]) > 0.0f ? r : 0.0f;
+                    o[e] = __bf16(r);
+                }
+                *reinterpret_cast<bf16x8*>(out + v * g.out_stride + co) = o;
+            }
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -892,6 +1094,10 @@ struct ConvLaunch {
     static constexpr bool HALO = TAPS == 27 && CIN % 32 == 0;
     static constexpr int BN_HALO = COUT <= 64 ? COUT : (COUT % 64 == 0 ? 64 : 48);
 
+    // the rows kernel
+    static constexpr bool ROWS = HALO && COUT % 32 == 0;
+    static constexpr int BN_ROWS = 32;
+
     template <int ACT, bool BIAS, bool OUTF32>
     static void fwd(const ConvGeom& g, const __bf16* in, const __bf16* w, const float* bias, void* out, hipStream_t s)
     {
@@ -908,9 +1114,34 @@ struct ConvLaunch {
                     while (NCHUNK % (2 * ks) == 0 && wgs * 2 * ks <= 512u &&
                            size_t(2 * ks) * g.nvox * COUT <= g.kpart_floats)
                         ks *= 2;
-                const dim3 grid(g.nvox / 256u, (COUT + BN_HALO - 1) / BN_HALO, ks);
-                hipLaunchKernelGGL((conv_fwd_halo<CIN, COUT, BN_HALO, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g,
-                                   in, w, bias, out);
+                // The rows kernel (8 x 64^3: 96 to 32 channels 626 -> 378 us, 192
+                // to 64 at 32^3 340 -> 202, 384 to 128 at 16^3 182 -> 105): BF16
+                // output at sides from 16, where a workgroup's block (32 x 4 x 4
+                // or 16 x 8 x 4 voxels) fits a sample, with rows that allow
+                // 16-byte accesses and 32-bit offsets into a sample.
+                bool rows = false;
+                if constexpr (ROWS && !OUTF32 && (ACT != ACT_NONE || !BIAS)) {
+                    const uint64_t sample_bytes = (uint64_t(1) << (3 * g.log_s)) * g.in_stride * 2u;
+                    const bool gated = ACT == ACT_RELU_GATE;
+                    const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out) | (gated ? uintptr_t(g.gate) : 0);
+                    const uint32_t strides = g.in_stride | g.out_stride | (gated ? g.gate_stride : 0u);
+                    rows = g.log_s >= 4 && sample_bytes < (uint64_t(1) << 32) && at % 16 == 0 && strides % 8 == 0;
+                    if (rows) {
+                        const dim3 grid(g.nvox / 512u * (COUT / BN_ROWS), ks);
+                        __bf16* o = static_cast<__bf16*>(out);
+                        if (g.log_s >= 5)
+                            hipLaunchKernelGGL((conv_fwd_rows<CIN, COUT, BN_ROWS, 2, 4, ACT, BIAS>), grid, dim3(256),
+                                               0, s, g, in, w, bias, o);
+                        else
+                            hipLaunchKernelGGL((conv_fwd_rows<CIN, COUT, BN_ROWS, 1, 8, ACT, BIAS>), grid, dim3(256),
+                                               0, s, g, in, w, bias, o);
+                    }
+                }
+                if (!rows) {
+                    const dim3 grid(g.nvox / 256u, (COUT + BN_HALO - 1) / BN_HALO, ks);
+                    hipLaunchKernelGGL((conv_fwd_halo<CIN, COUT, BN_HALO, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g,
+                                       in, w, bias, out);
+                }
                 if (ks > 1) {
                     const uint64_t n = uint64_t(g.nvox) * (COUT / 4);
                     hipLaunchKernelGGL((conv_ksplit_sum<ACT, BIAS, OUTF32>), dim3(uint32_t((n + 255) / 256)), dim3(256),
