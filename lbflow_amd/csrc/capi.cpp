@@ -17,6 +17,7 @@
 
 #include "../../include/lbflow.h"
 #include "device.h"
+#include "host_copy.h"
 #include "operator_f64.h"
 #include "setup.h"
 
@@ -85,6 +86,7 @@ struct lbf_ctx {
     bool has_prev = false;
     uint64_t dev_bytes = 0;
     std::vector<void*> allocations;
+    std::shared_ptr<HostStage> stage;   // large copies to the host (host_copy.h)
     std::string err;
     std::string kernel_name;
 };
@@ -866,9 +868,9 @@ int lbf_fields(lbf_ctx* c, double* rho0, double* rho1, double* u)
 {
     if (!c) return -1;
     HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    if (rho0) HIP_CHECK(c, hipMemcpy(rho0, c->d_rho0, c->N * 8, hipMemcpyDeviceToHost));
-    if (rho1 && c->NP == 2) HIP_CHECK(c, hipMemcpy(rho1, c->d_rho1, c->N * 8, hipMemcpyDeviceToHost));
-    if (u) HIP_CHECK(c, hipMemcpy(u, c->d_u, size_t(c->D) * c->N * 8, hipMemcpyDeviceToHost));
+    if (rho0) HIP_CHECK(c, copy_to_host(c->stage, rho0, c->d_rho0, c->N * 8, c->stream));
+    if (rho1 && c->NP == 2) HIP_CHECK(c, copy_to_host(c->stage, rho1, c->d_rho1, c->N * 8, c->stream));
+    if (u) HIP_CHECK(c, copy_to_host(c->stage, u, c->d_u, size_t(c->D) * c->N * 8, c->stream));
     return 0;
 }
 
@@ -879,7 +881,7 @@ int lbf_get_populations(lbf_ctx* c, double* out)
     const size_t planes = size_t(c->NP) * c->Q;
     const size_t n = c->pop_elems;
     if (c->elem == 8 && c->layout == 0) {
-        HIP_CHECK(c, hipMemcpy(out, c->f[c->cur], n * 8, hipMemcpyDeviceToHost));
+        HIP_CHECK(c, copy_to_host(c->stage, out, c->f[c->cur], n * 8, c->stream));
         return 0;
     }
     std::vector<double> h64(c->elem == 8 ? n : 0);

@@ -279,6 +279,16 @@ __global__ void net_to_bf16(const float* __restrict__ p, uint32_t n, __bf16* __r
     if (i < n) pb[i] = __bf16(p[i]);
 }
 
+// A layer in the caller's layout: out = W[rows][k] (rows of pitch kp), then bias[rows].
+__global__ void __launch_bounds__(256)
+net_flatten(const float* __restrict__ w, const float* __restrict__ b, uint32_t rows, uint32_t k, uint32_t kp,
+            float* __restrict__ out)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x, n = rows * k;
+    if (i < n) out[i] = w[size_t(i / k) * kp + i % k];
+    else if (i < n + rows) out[i] = b[i - n];
+}
+
 // wt[ci][tap' * cout + co] = w[co][tap * cin + ci], tap' = taps - 1 - tap (mirrored
 // offset), both zero-padded to their KP.
 __global__ void net_transpose_w(const __bf16* __restrict__ w, uint32_t cin, uint32_t cout, uint32_t taps,
@@ -368,6 +378,12 @@ hipError_t launch_net_head_fields(const float* out16, const uint8_t* mask, uint3
 hipError_t launch_net_to_bf16(const float* p, uint32_t n, __bf16* pb, hipStream_t s)
 {
     hipLaunchKernelGGL(net_to_bf16, grid_for(n), dim3(256), 0, s, p, n, pb);
+    return hipGetLastError();
+}
+hipError_t launch_net_flatten(const float* w, const float* b, uint32_t rows, uint32_t k, uint32_t kp, float* out,
+                              hipStream_t s)
+{
+    hipLaunchKernelGGL(net_flatten, grid_for(uint64_t(rows) * k + rows), dim3(256), 0, s, w, b, rows, k, kp, out);
     return hipGetLastError();
 }
 hipError_t launch_net_transpose_w(const __bf16* w, uint32_t cin, uint32_t cout, uint32_t taps, uint32_t kp,

@@ -24,6 +24,7 @@
 
 #include "../../include/lbflow.h"
 #include "conv_types.h"
+#include "host_copy.h"
 
 namespace lbf {
 uint32_t conv_wgrad_splits(int cin, int cout, int taps, uint32_t nvox);
@@ -49,6 +50,8 @@ hipError_t launch_net_head4(const float* out16, uint32_t nvox, float* out4, hipS
 hipError_t launch_net_head_fields(const float* out16, const uint8_t* mask, uint32_t nvox, const float* scale,
                                   const float* offset, float* out4, hipStream_t s);
 hipError_t launch_net_to_bf16(const float* p, uint32_t n, __bf16* pb, hipStream_t s);
+hipError_t launch_net_flatten(const float* w, const float* b, uint32_t rows, uint32_t k, uint32_t kp, float* out,
+                              hipStream_t s);
 hipError_t launch_net_transpose_w(const __bf16* w, uint32_t cin, uint32_t cout, uint32_t taps, uint32_t kp,
                                   uint32_t kpt, __bf16* wt, hipStream_t s);
 }  // namespace lbf
@@ -73,6 +76,7 @@ constexpr int kLayers[NLAYERS][4] = {
 struct Layer {
     int cin = 0, cout = 0, taps = 0, level = 0, real_out = 0;
     uint32_t kp = 0, kpt = 0;
+    uint64_t flat = 0;                         // first parameter in the caller's layout
     float *w = nullptr, *b = nullptr;          // FP32 master [cout][kp], [cout]
     float *gw = nullptr, *gb = nullptr;
     float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
@@ -97,6 +101,8 @@ struct lbf_net {
     float* kpart;                  // forward split over input channels: FP32 partials
     double *lpart, *loss;
     size_t wpart_floats = 0;
+    float* flat = nullptr;         // parameters or gradients in the caller's layout
+    std::shared_ptr<HostStage> stage;   // large copies to the host (host_copy.h)
     // warm starts: capacity pore masks and their physical fields, allocated on first use
     uint8_t* warm_mask = nullptr;
     float* warm_fields = nullptr;
@@ -328,6 +334,7 @@ int lbf_net_create(uint32_t side, uint32_t capacity, uint64_t seed, lbf_net** ou
         l.kp = uint32_t(conv_kp(l.cin, l.taps));
         l.kpt = uint32_t(conv_kp(l.cout, l.taps));
         const size_t nw = size_t(l.cout) * l.kp;
+        if (i) l.flat = n->L[i - 1].flat + real_params(n->L[i - 1]);
         rc |= nalloc(n, &l.w, nw);
         rc |= nalloc(n, &l.gw, nw);
         rc |= nalloc(n, &l.mw, nw);
@@ -389,6 +396,7 @@ int lbf_net_create(uint32_t side, uint32_t capacity, uint64_t seed, lbf_net** ou
         rc |= nalloc(n, &n->kpart, KPART_FLOATS);
         rc |= nalloc(n, &n->lpart, size_t(v[0] / 256 + 1));
         rc |= nalloc(n, &n->loss, 1);
+        rc |= nalloc(n, &n->flat, size_t(lbf_net_param_count(n)));
     }
     if (rc || refresh_bf16(n) || hipStreamSynchronize(n->stream) != hipSuccess) {
         std::string e = n->err.empty() ? "HIP error while creating the network" : n->err;
@@ -410,16 +418,9 @@ uint64_t lbf_net_param_count(const lbf_net* n)
 int lbf_net_get_params(lbf_net* n, float* host)
 {
     if (!n || !host) return -1;
-    NHIP(n, hipStreamSynchronize(n->stream));
-    float* o = host;
-    for (const Layer& l : n->L) {
-        std::vector<float> w(size_t(l.cout) * l.kp), b(l.cout);
-        NHIP(n, hipMemcpy(w.data(), l.w, w.size() * 4, hipMemcpyDeviceToHost));
-        NHIP(n, hipMemcpy(b.data(), l.b, b.size() * 4, hipMemcpyDeviceToHost));
-        for (int co = 0; co < l.real_out; ++co)
-            for (int k = 0; k < l.taps * l.cin; ++k) *o++ = w[size_t(co) * l.kp + k];
-        for (int co = 0; co < l.real_out; ++co) *o++ = b[co];
-    }
+    for (const Layer& l : n->L)
+        NHIP(n, launch_net_flatten(l.w, l.b, l.real_out, l.taps * l.cin, l.kp, n->flat + l.flat, n->stream));
+    NHIP(n, copy_to_host(n->stage, host, n->flat, lbf_net_param_count(n) * sizeof(float), n->stream));
     return 0;
 }
 
@@ -489,15 +490,9 @@ int lbf_net_gradients(lbf_net* n, const uint8_t* mask, const float* target, uint
     if (!n || !mask || !target || !weights) return -1;
     if (loss_and_grad(n, mask, target, count, weights, loss)) return -1;
     if (grad_host) {
-        float* o = grad_host;
-        for (const Layer& l : n->L) {
-            std::vector<float> w(size_t(l.cout) * l.kp), b(l.cout);
-            NHIP(n, hipMemcpy(w.data(), l.gw, w.size() * 4, hipMemcpyDeviceToHost));
-            NHIP(n, hipMemcpy(b.data(), l.gb, b.size() * 4, hipMemcpyDeviceToHost));
-            for (int co = 0; co < l.real_out; ++co)
-                for (int k = 0; k < l.taps * l.cin; ++k) *o++ = w[size_t(co) * l.kp + k];
-            for (int co = 0; co < l.real_out; ++co) *o++ = b[co];
-        }
+        for (const Layer& l : n->L)
+            NHIP(n, launch_net_flatten(l.gw, l.gb, l.real_out, l.taps * l.cin, l.kp, n->flat + l.flat, n->stream));
+        NHIP(n, copy_to_host(n->stage, grad_host, n->flat, lbf_net_param_count(n) * sizeof(float), n->stream));
     }
     return 0;
 }
