@@ -650,6 +650,73 @@ conv_fwd_coarse(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restr
 }
 
 // ---------------------------------------------------------------------------
+// forward (and input gradient), 3x3x3 with Cin a multiple of 32, few voxels at
+// sides from 8: one wave per 16 output channels, tile of 16 voxels and split of
+// the input channels, the 27 taps of a 32-channel chunk in flight, in the halo
+// and rows kernels' order of k (chunks, then taps).  Latency bound; those
+// kernels' 256-voxel workgroups leave most of the chip idle here.
+// ---------------------------------------------------------------------------
+template <int CIN, int COUT, int ACT, bool BIAS, bool OUTF32>
+__global__ void __launch_bounds__(64, 1)
+conv_fwd_few(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restrict__ w,
+             const float* __restrict__ bias, void* __restrict__ out)
+{
+    constexpr int KP = conv_kp(CIN, 27);
+    static_assert(CIN % 32 == 0 && COUT % 16 == 0, "shape");
+    const int r16 = threadIdx.x & 15, grp = threadIdx.x >> 4;
+    const uint32_t vbase = blockIdx.x * 16u;   // nvox is a multiple of 512
+    const int co = int(blockIdx.y) * 16 + r16;
+    const int chunks = (CIN / 32) / int(gridDim.z), c0 = int(blockIdx.z) * chunks * 32;
+    const uint32_t ls = g.log_s, m = (1u << ls) - 1u;
+    const __bf16* wp = w + size_t(co) * KP + 8 * grp + c0;
+    const __bf16* ip = in + 8 * grp + c0;
+    // the voxel's neighbours along each axis, as summands of their index
+    uint32_t xs[3], ys[3], zs[3];
+    const uint32_t v0 = vbase + r16;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        xs[d] = (v0 + uint32_t(d) - 1u) & m;
+        ys[d] = (((v0 >> ls) + uint32_t(d) - 1u) & m) << ls;
+        zs[d] = ((((v0 >> (2 * ls)) + uint32_t(d) - 1u) & m) << (2 * ls)) | (v0 >> (3 * ls) << (3 * ls));
+    }
+    bf16x8 a[27], b[27];
+    auto request = [&](int tap) __attribute__((always_inline)) {
+        b[tap] = *reinterpret_cast<const bf16x8*>(wp + tap * CIN);
+        a[tap] = *reinterpret_cast<const bf16x8*>(ip + size_t(zs[tap / 9] + ys[tap / 3 % 3] + xs[tap % 3]) * g.in_stride);
+    };
+    f32x4 acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < 27; ++t) request(t);
+#pragma unroll 1
+    for (int c = 1; c <= chunks; ++c) {
+        wp += 32;
+        ip += 32;
+        const bool more = c < chunks;
+#pragma unroll
+        for (int t = 0; t < 27; ++t) {
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[t], acc, 0, 0, 0);
+            if (more) request(t);
+        }
+    }
+    const float bb = BIAS ? bias[co] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const uint32_t v = vbase + 4u * grp + r;
+        float x = acc[r];
+        if (gridDim.z > 1) {
+            // split: this split's FP32 partial, summed by conv_ksplit_sum
+            g.kpart[(size_t(blockIdx.z) * g.nvox + v) * COUT + co] = x;
+            continue;
+        }
+        x += bb;
+        if (ACT == ACT_RELU) x = x > 0.0f ? x : 0.0f;
+        if (ACT == ACT_RELU_GATE) x = float(g.gate[size_t(v) * g.gate_stride + co]) > 0.0f ? x : 0.0f;
+        if (OUTF32) static_cast<float*>(out)[size_t(v) * g.out_stride + co] = x;
+        else static_cast<__bf16*>(out)[size_t(v) * g.out_stride + co] = __bf16(x);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // weight gradient
 // ---------------------------------------------------------------------------
 template <int CIN, int COUT, int TAPS, int BM, int BN>
@@ -1203,12 +1270,21 @@ struct ConvLaunch {
                 // or 16 x 8 x 4 voxels) fits a sample, with rows that allow
                 // 16-byte accesses and 32-bit offsets into a sample.
                 bool rows = false;
+                // Few voxels: a wave of the kernel for them per 16 x 16 results and
+                // split, up to one wave per SIMD (per call with its 10 us: 384 to
+                // 128 channels at 8^3 58 -> 36 us, 128 to 128 31 -> 24, 32 to 32 at
+                // 16^3 20 -> 15; at twice as many waves 31.6 -> 30.5 and 25.9 -> 29,
+                // beyond that the other two are faster).
+                const bool few = (g.nvox / 16u) * (COUT / 16u) * ks <= 1024u;
+                if (few)
+                    hipLaunchKernelGGL((conv_fwd_few<CIN, COUT, ACT, BIAS, OUTF32>),
+                                       dim3(g.nvox / 16u, COUT / 16, ks), dim3(64), 0, s, g, in, w, bias, out);
                 if constexpr (ROWS && !OUTF32 && (ACT != ACT_NONE || !BIAS)) {
                     const uint64_t sample_bytes = (uint64_t(1) << (3 * g.log_s)) * g.in_stride * 2u;
                     const bool gated = ACT == ACT_RELU_GATE;
                     const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out) | (gated ? uintptr_t(g.gate) : 0);
                     const uint32_t strides = g.in_stride | g.out_stride | (gated ? g.gate_stride : 0u);
-                    rows = g.log_s >= 4 && sample_bytes < (uint64_t(1) << 32) && at % 16 == 0 && strides % 8 == 0;
+                    rows = !few && g.log_s >= 4 && sample_bytes < (uint64_t(1) << 32) && at % 16 == 0 && strides % 8 == 0;
                     if (rows) {
                         const dim3 grid(g.nvox / 512u * (COUT / BN_ROWS), ks);
                         __bf16* o = static_cast<__bf16*>(out);
@@ -1220,7 +1296,7 @@ struct ConvLaunch {
                                                0, s, g, in, w, bias, o);
                     }
                 }
-                if (!rows) {
+                if (!rows && !few) {
                     const dim3 grid(g.nvox / 256u, (COUT + BN_HALO - 1) / BN_HALO, ks);
                     hipLaunchKernelGGL((conv_fwd_halo<CIN, COUT, BN_HALO, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g,
                                        in, w, bias, out);
