@@ -111,23 +111,6 @@ __device__ __forceinline__ int wrap(int c, int n)
     return c < 0 ? c + n : (c >= n ? c - n : c);
 }
 
-// Pull source of direction q at (x,y,z) for lattice Q (components slowest first).
-template <int Q>
-__device__ __forceinline__ uint32_t pull_source(const GridDev& g, int x, int y, int z, int q)
-{
-    using L = Lattice<Q>;
-    int ex, ey, ez;
-    if constexpr (Q == 9) {
-        ez = 0; ey = L::e[q][0]; ex = L::e[q][1];
-    } else {
-        ez = L::e[q][0]; ey = L::e[q][1]; ex = L::e[q][2];
-    }
-    const int xs = ex ? wrap(x - ex, int(g.nx)) : x;
-    const int ys = ey ? wrap(y - ey, int(g.ny)) : y;
-    const int zs = ez ? wrap(z - ez, int(g.nz)) : z;
-    return uint32_t(zs) * g.nxy + uint32_t(ys) * g.nx + uint32_t(xs);
-}
-
 // Neighbour x + e_q (gradient stencil).
 template <int Q>
 __device__ __forceinline__ uint32_t push_target(const GridDev& g, int x, int y, int z, int q)

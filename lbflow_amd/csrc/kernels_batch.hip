@@ -91,13 +91,13 @@ __device__ __forceinline__ void batch_site(const BatchParams& p, const float* __
         for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.S + slot] = u[d];
     }
     collide_f32<Q, MRT>(h, drho, u, F, p.relax);
-    bool finite = true;
+    float chk = 0.0f;   // stays 0 while every population is finite
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        finite = finite && isfinite(h[q]);
+        chk = fmaf(h[q], 0.0f, chk);
         st_pop<true>(fout, base + pop_index<Q, true, O>(0u, q, local), h[q]);
     }
-    if (!finite) raise_status(status, 4, p.t);
+    if (chk != 0.0f) raise_status(status, 4, p.t);
 }
 
 // Persistent step over the active tiles.  The work unit is UNIT slots of one
@@ -122,10 +122,9 @@ batch_step(BatchParams p, const float* __restrict__ fin, float* __restrict__ fou
 #pragma unroll
         for (uint32_t j = 0; j < UNIT; j += BS) {
             const uint32_t slot = tile * TILE + (k % PER_TILE) * UNIT + j + threadIdx.x;
-            const uint32_t s = site[slot];
+            const uint32_t s = site[slot], dsc = desc[slot];   // one wait for both
             if (s != NO_SITE)
-                batch_site<Q, MRT, INIT, O>(p, fin, fout, cr, slot, s, desc[slot], rank, lab, ucur, uadj, upres,
-                                            status);
+                batch_site<Q, MRT, INIT, O>(p, fin, fout, cr, slot, s, dsc, rank, lab, ucur, uadj, upres, status);
         }
     }
 }

@@ -61,11 +61,11 @@ __device__ __forceinline__ bool resolve32(const ColorArgs& a, uint32_t& site, ui
 // PB/VB sites apply the Zou-He boundary to the pulled populations and return
 // its density deviation and velocity in dzh / uzh.
 struct NoPre {
-    template <typename O> __device__ void operator()(const O*) const {}
+    __device__ void operator()(const uint32_t*) const {}
 };
 
-// PRE (sparse): called with the pull offsets before the populations are
-// loaded (the step issues its indicator gathers there).
+// PRE (sparse): called with the slots that the pull reads, before the
+// populations are loaded (the step issues its indicator gathers there).
 template <int Q, bool INIT, int LAYOUT, typename O, bool OWN = false, typename PRE = NoPre>
 __device__ __forceinline__ void load_color32(const ColorArgs& a, uint32_t site, uint32_t slot, uint32_t desc,
                                              const DevLabel& lab, float* h, float* f0, double& r0, double& dr,
@@ -90,9 +90,10 @@ __device__ __forceinline__ void load_color32(const ColorArgs& a, uint32_t site, 
         if constexpr (LAYOUT == SPARSE && !std::is_same<PRE, NoPre>::value) {
             // only the neighbours' offsets (the populations are set, not pulled)
             O off[Q];
+            uint32_t from[Q];
             pull_offsets<Q, LAYOUT, O, true, 2 * Q>(a.rank, desc & DESC_LINK_MASK, slot, make_stencil(a.g, site),
-                                                    a.g.nx, a.P, off);
-            pre(off);
+                                                    a.g.nx, a.P, off, from);
+            pre(from);
         }
         // colorfluid.cpp:214-236: f[phase] = ai_phase rho_phase - 1.5 w (e.F), other phase 0
         const int ph = lab.phase;
@@ -112,8 +113,9 @@ __device__ __forceinline__ void load_color32(const ColorArgs& a, uint32_t site, 
     const Stencil stn = make_stencil(a.g, site);
     O off[Q];
     off[0] = pop_index<2 * Q, BLK, O>(a.P, 0, slot);
-    pull_offsets<Q, LAYOUT, O, BLK, 2 * Q>(a.rank, desc & DESC_LINK_MASK, slot, stn, a.g.nx, uint32_t(P), off);
-    pre(off);
+    uint32_t from[Q];
+    pull_offsets<Q, LAYOUT, O, BLK, 2 * Q>(a.rank, desc & DESC_LINK_MASK, slot, stn, a.g.nx, uint32_t(P), off, from);
+    pre(from);
     // The boundary path is chosen before the loads, so that plain sites can
     // fold their populations into the sums as they arrive.
     const bool film_links = desc & DESC_FILM;
@@ -380,7 +382,8 @@ __global__ void __launch_bounds__(256) color_density_f32(ColorArgs a)
     if (!resolve32<LAYOUT>(a, site, slot)) return;
     const uint32_t desc = a.desc[slot];
     const DevLabel& lab = a.lab[desc >> DESC_LABEL_SHIFT];
-    if (!(lab.kind & KIND_FLUID)) return;
+    // sparse: every slot is a fluid site, see scsp_step_f32
+    if (LAYOUT != SPARSE && !(lab.kind & KIND_FLUID)) return;
     float h[Q], f0[Q], dzh, uzh[Lattice<Q>::D];
     double r0, dr;
     load_color32<Q, INIT, LAYOUT, O, OWN>(a, site, slot, desc, lab, h, f0, r0, dr, dzh, uzh);
@@ -405,7 +408,7 @@ __global__ void __launch_bounds__(256) color_step_f32(ColorArgs a)
     const uint32_t desc = a.desc[slot];
     const DevLabel& lab = a.lab[desc >> DESC_LABEL_SHIFT];
     const int kind = lab.kind;
-    if (!(kind & KIND_FLUID)) return;
+    if (LAYOUT != SPARSE && !(kind & KIND_FLUID)) return;
 
     float h[Q], f0[Q], dzh = 0.0f, uzh[D];
     double r0d, drd;
@@ -421,18 +424,17 @@ __global__ void __launch_bounds__(256) color_step_f32(ColorArgs a)
         // formed once both have arrived: one memory round trip for the site
         // (a gradient formed before the population loads waited on its own
         // gathers and on the wall entry first).  Neighbour x + e_q is the
-        // pull source of op(q), its slot recovered from the blocked offset
-        // (block, lane); solid where link q bounces back.
+        // pull source of op(q), solid where link q bounces back (its own slot
+        // is read then: a branch per neighbour split the gathers).
         const uint32_t links = desc & DESC_LINK_MASK;
         const int32_t wi = a.wall_slot[slot];
         float dn[Q];
-        auto gather = [&](const O* off) __attribute__((always_inline)) {
+        auto gather = [&](const uint32_t* from) __attribute__((always_inline)) {
             dn[0] = a.dens_slot[slot];
 #pragma unroll
             for (int q = 1; q < Q; ++q) {
-                const O o = off[L::op[q]];
-                const uint32_t m = (uint32_t(o / O(2 * Q * 64)) << 6) | uint32_t(o & O(63));
-                dn[q] = ((links >> q) & 1u) ? SOLID_N32 : a.dens_slot[m];
+                const float v = a.dens_slot[from[L::op[q]]];
+                dn[q] = ((links >> q) & 1u) ? SOLID_N32 : v;
             }
         };
         load_color32<Q, INIT, LAYOUT, O, OWN>(a, i, slot, desc, lab, h, f0, r0d, drd, dzh, uzh, gather);
@@ -640,7 +642,8 @@ __global__ void __launch_bounds__(256) color_step_f32(ColorArgs a)
     // that sum the phase-0 mass grew by a factor 1 + 1.5e-8 per step).
     const double dens0T64 = r0d / rtd;
     const float dens0T = float(dens0T64);
-    bool finite = true;
+    // one set of stores for both kinds of site: with a set in each branch a wave
+    // at the edge of an interface wrote every line in two parts
     if (norm > 1e-9f) {
         const float b01 = a.betaf * dens0T * r1 * inv_rt;
         const float akn = a.akf * norm / tau;
@@ -657,21 +660,20 @@ __global__ void __launch_bounds__(256) color_step_f32(ColorArgs a)
             if constexpr (!CSF) h[q] += akn * (float(L::w[q]) * angle * angle - a.bif[q]);
             if (L::diagonal(q)) angle *= (1.0f / SQRT2_32);
             const float feq0 = r0 * a.ai0f[q] + r1 * a.ai1f[q];
-            const float fo = float(fma(dens0T64, double(h[q]) + a.dist0r[q], double(b01 * angle * feq0)));
-            finite = finite && isfinite(h[q]) && isfinite(fo);
-            st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, q, slot), h[q]);
-            st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, Q + q, slot), fo);
+            f0[q] = float(fma(dens0T64, double(h[q]) + a.dist0r[q], double(b01 * angle * feq0)));
         }
     } else {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) {
-            const float fo = float(dens0T64 * (double(h[q]) + a.dist0r[q]));
-            finite = finite && isfinite(h[q]) && isfinite(fo);
-            st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, q, slot), h[q]);
-            st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, Q + q, slot), fo);
-        }
+        for (int q = 0; q < Q; ++q) f0[q] = float(dens0T64 * (double(h[q]) + a.dist0r[q]));
     }
-    if (!finite) raise_status(a.status, 4, a.t);
+    float chk = 0.0f;   // stays 0 while every population is finite
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        chk = fmaf(f0[q], 0.0f, fmaf(h[q], 0.0f, chk));
+        st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, q, slot), h[q]);
+        st_pop<LAYOUT == SPARSE>(a.fout32, pop_index<2 * Q, LAYOUT == SPARSE, O>(a.P, Q + q, slot), f0[q]);
+    }
+    if (chk != 0.0f) raise_status(a.status, 4, a.t);
 }
 
 // wallGradient tanh at the wall sites (colorfluid.cpp:494-518), from the FP32

@@ -109,7 +109,7 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
     const uint32_t dsc = desc[LAYOUT == SPARSE ? slot : i];
     const DevLabel* lb = lab + (dsc >> DESC_LABEL_SHIFT);
     const int kind = lb->kind;
-    const bool fluid = kind & KIND_FLUID;
+    const bool fluid = LAYOUT == SPARSE || (kind & KIND_FLUID);   // see the FP32 kernel
     if (!fluid && (INIT || LAYOUT != DENSE_ALL)) return;
     double f[Q];
     if (!INIT) {
@@ -270,7 +270,9 @@ scsp_step_f32(ScspParams p, const float* __restrict__ fin, float* __restrict__ f
     constexpr bool BLK = LAYOUT == SPARSE;   // sparse: blocks of 64 slots
     const uint32_t dsc = desc[LAYOUT == SPARSE ? slot : i];
     const LabelF lb = lab[dsc >> DESC_LABEL_SHIFT];
-    const bool fluid = lb.kind & KIND_FLUID;
+    // sparse: every slot is a fluid site; a test of its label here would put the
+    // label's load between those of the descriptor and the rank index
+    const bool fluid = LAYOUT == SPARSE || (lb.kind & KIND_FLUID);
     if (!fluid && (INIT || LAYOUT != DENSE_ALL)) return;
     float h[Q];
     if (!INIT) {
