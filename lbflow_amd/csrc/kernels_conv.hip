@@ -1179,6 +1179,22 @@ conv_wgrad_rows(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restr
     }
 }
 
+// s += p[0] + p[stride] + .. in order, the loads of 16 summands in flight
+__device__ __forceinline__ float sum_in_order(const float* __restrict__ p, uint32_t count, size_t stride)
+{
+    float s = 0.0f;
+    uint32_t k = 0;
+    for (; k + 16 <= count; k += 16) {
+        float x[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = p[(k + j) * stride];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s += x[j];
+    }
+    for (; k < count; ++k) s += p[k * stride];
+    return s;
+}
+
 // dW[i] = sum over splits of partial[s][i] in a fixed order (deterministic).
 // Up to 64 splits: in split order.  More: the splits are summed in groups of
 // SPLIT_GROUP consecutive ones in parallel (each group's sum stored in the
@@ -1192,42 +1208,39 @@ sum_split_groups(float* __restrict__ partial, uint32_t n, uint32_t splits)
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
     const uint32_t k0 = blockIdx.y * SPLIT_GROUP, k1 = k0 + SPLIT_GROUP < splits ? k0 + SPLIT_GROUP : splits;
-    float s = 0.0f;
-    for (uint32_t k = k0; k < k1; ++k) s += partial[size_t(k) * n + i];
-    partial[size_t(k0) * n + i] = s;
+    partial[size_t(k0) * n + i] = sum_in_order(partial + size_t(k0) * n + i, k1 - k0, n);
 }
 
+// The last cblocks workgroups sum the bias partials: db[c] = sum over splits of
+// bpart[split][c], in split order (a kernel of their own with a load per
+// summand in flight took 27 us a layer, as long as the rest of these sums).
 __global__ void __launch_bounds__(256)
-sum_splits(const float* __restrict__ partial, uint32_t n, uint32_t splits, uint32_t step, float* __restrict__ out)
+sum_splits(const float* __restrict__ partial, uint32_t n, uint32_t splits, uint32_t step, float* __restrict__ out,
+           const float* __restrict__ bpart, uint32_t cout, uint32_t bsplits, uint32_t cblocks, float* __restrict__ db)
 {
+    const uint32_t wblocks = gridDim.x - cblocks;
+    if (blockIdx.x >= wblocks) {
+        const uint32_t c = (blockIdx.x - wblocks) * 256u + threadIdx.x;
+        if (c < cout) db[c] = sum_in_order(bpart + c, bsplits, cout);
+        return;
+    }
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n) return;
-    float s = 0.0f;
-    for (uint32_t k = 0; k < splits; k += step) s += partial[size_t(k) * n + i];
-    out[i] = s;
+    out[i] = sum_in_order(partial + i, (splits + step - 1) / step, size_t(step) * n);
 }
 
-// db[c] = sum over splits of bpart[split][c], in split order.
-__global__ void __launch_bounds__(256)
-sum_bias_splits(const float* __restrict__ bpart, uint32_t cout, uint32_t splits, float* __restrict__ db)
+static void launch_sum_splits(float* partial, uint32_t n, uint32_t splits, float* dw, const float* bpart,
+                              uint32_t cout, float* db, hipStream_t s)
 {
-    const uint32_t c = blockIdx.x * 256u + threadIdx.x;
-    if (c >= cout) return;
-    float s = 0.0f;
-    for (uint32_t k = 0; k < splits; ++k) s += bpart[size_t(k) * cout + c];
-    db[c] = s;
-}
-
-static void launch_sum_splits(float* partial, uint32_t n, uint32_t splits, float* dw, hipStream_t s)
-{
-    const uint32_t blocks = (n + 255) / 256;
+    const uint32_t blocks = (n + 255) / 256, cblocks = db ? (cout + 255) / 256 : 0;
+    uint32_t step = 1;
     if (splits > 64) {
         hipLaunchKernelGGL(sum_split_groups, dim3(blocks, (splits + SPLIT_GROUP - 1) / SPLIT_GROUP), dim3(256), 0, s,
                            partial, n, splits);
-        hipLaunchKernelGGL(sum_splits, dim3(blocks), dim3(256), 0, s, partial, n, splits, SPLIT_GROUP, dw);
-    } else {
-        hipLaunchKernelGGL(sum_splits, dim3(blocks), dim3(256), 0, s, partial, n, splits, 1u, dw);
+        step = SPLIT_GROUP;
     }
+    hipLaunchKernelGGL(sum_splits, dim3(blocks + cblocks), dim3(256), 0, s, partial, n, splits, step, dw, bpart, cout,
+                       splits, cblocks, db);
 }
 
 // ---------------------------------------------------------------------------
@@ -1358,17 +1371,14 @@ struct ConvLaunch {
                 else
                     hipLaunchKernelGGL((conv_wgrad_halo<CIN, COUT>), dim3((CIN / 16) * (COUT / 32) * splits),
                                        dim3(256), 0, s, g, in, dz, partial, per, bp);
-                launch_sum_splits(partial, uint32_t(COUT) * KP, splits, dw, s);
-                if (db)
-                    hipLaunchKernelGGL(sum_bias_splits, dim3((COUT + 255) / 256), dim3(256), 0, s, bpart,
-                                       uint32_t(COUT), splits, db);
+                launch_sum_splits(partial, uint32_t(COUT) * KP, splits, dw, bpart, COUT, db, s);
                 return;
             }
         }
         const uint32_t per = ((g.nvox + splits - 1) / splits + 127u) / 128u * 128u;
         const dim3 grid((KP + BN_W - 1) / BN_W, (COUT + BM_W - 1) / BM_W, splits);
         hipLaunchKernelGGL((conv_wgrad<CIN, COUT, TAPS, BM_W, BN_W>), grid, dim3(256), 0, s, g, in, dz, partial, per);
-        launch_sum_splits(partial, uint32_t(COUT) * KP, splits, dw, s);
+        launch_sum_splits(partial, uint32_t(COUT) * KP, splits, dw, nullptr, COUT, nullptr, s);
     }
 };
 
