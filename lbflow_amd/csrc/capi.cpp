@@ -22,6 +22,8 @@
 #include "setup.h"
 
 namespace lbf {
+hipError_t launch_scsp_steps(int Q, bool mrt, int layout, uint32_t steps, const ScspParams& p, const ScspBuffers& b,
+                             hipStream_t s);
 hipError_t launch_scsp(int Q, bool mrt, bool init, bool fp32, int layout, const ScspParams& p,
                        const ScspBuffers& b, hipStream_t s);
 hipError_t launch_color(int Q, bool mrt, bool init, bool stream_solids, const ColorArgs& a, hipStream_t s);
@@ -815,6 +817,31 @@ static int run_step(lbf_ctx* c, bool init, uint32_t flags)
     return 0;
 }
 
+// n plain steps.  Small FP64 single-phase lattices take several per launch; the
+// chunk bounds a launch's length (a few ms).  The populations end in the
+// buffer in which single steps would leave them.
+static int advance_steps(lbf_ctx* c, uint64_t n)
+{
+    constexpr uint64_t CHUNK = 512;
+    if (c->NP == 1 && c->elem == 8 && c->layout != 2 && c->N > 0 && c->N <= scsp_few_sites(c->Q)) {
+        while (n > 1) {
+            const uint32_t steps = uint32_t(std::min(n, CHUNK));
+            ScspParams p = scsp_params(c, 0u);
+            p.t = c->t + 1;
+            ScspBuffers b = scsp_buffers(c, false);
+            if (steps % 2 == 0) b.fout = c->f[c->cur];
+            const hipError_t e = launch_scsp_steps(c->Q, c->d.equil == LBF_MRT, c->layout, steps, p, b, c->stream);
+            if (e != hipSuccess) return fail(c, std::string("HIP error: kernel launch: ") + hipGetErrorString(e));
+            c->cur ^= int(steps % 2);
+            c->t += steps;
+            n -= steps;
+        }
+    }
+    for (uint64_t k = 0; k < n; ++k)
+        if (run_step(c, false, 0u)) return -1;
+    return 0;
+}
+
 int lbf_init(lbf_ctx* c)
 {
     if (!c) return -1;
@@ -838,9 +865,7 @@ int lbf_step(lbf_ctx* c, uint32_t flags)
 int lbf_advance(lbf_ctx* c, uint64_t n)
 {
     if (!c) return -1;
-    for (uint64_t k = 0; k < n; ++k)
-        if (run_step(c, false, 0u)) return -1;
-    return 0;
+    return advance_steps(c, n);
 }
 
 uint64_t lbf_time(const lbf_ctx* c) { return c ? c->t : 0; }
@@ -1086,8 +1111,7 @@ int lbf_timed_advance(lbf_ctx* c, uint64_t n, double* ms)
     HIP_CHECK(c, hipEventCreate(&e0));
     HIP_CHECK(c, hipEventCreate(&e1));
     HIP_CHECK(c, hipEventRecord(e0, c->stream));
-    for (uint64_t k = 0; k < n; ++k)
-        if (run_step(c, false, 0u)) return -1;
+    if (advance_steps(c, n)) return -1;
     HIP_CHECK(c, hipEventRecord(e1, c->stream));
     HIP_CHECK(c, hipEventSynchronize(e1));
     float f = 0.0f;

@@ -152,6 +152,10 @@ struct LabelF {
     float pad;
 };
 
+// Lattices up to this many sites step several times per launch (FP64, dense):
+// the largest workgroup whose threads keep their registers.
+constexpr uint32_t scsp_few_sites(int Q) { return Q == 9 ? 1024u : 512u; }
+
 // Scalar parameters of the single-phase step kernels (by value).
 struct ScspParams {
     GridDev g;

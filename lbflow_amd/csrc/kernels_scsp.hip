@@ -77,6 +77,135 @@ __device__ __forceinline__ bool resolve(const ScspParams& p, const uint32_t* __r
     return true;
 }
 
+// Macro variables, boundary and collision of one fluid site from its pulled
+// populations.
+template <int Q, bool MRT, bool INIT>
+__device__ __forceinline__ void scsp_site_f64(const ScspParams& p, const DevLabel& lb, uint32_t dsc, uint32_t i,
+                                              unsigned long long t, const double* __restrict__ A4,
+                                              const double* __restrict__ B4, double* __restrict__ rho_out,
+                                              double* __restrict__ u_out, double* __restrict__ uadj,
+                                              DevStatus* __restrict__ status, const DevZouHe* __restrict__ zh, double* f)
+{
+#pragma clang fp contract(off)
+    using L = Lattice<Q>;
+    constexpr int D = L::D;
+    const int kind = lb.kind;
+    const double force[3] = {lb.force[0], lb.force[1], D == 3 ? lb.force[2] : 0.0};
+    const bool forced = kind & KIND_FORCED;
+    if (INIT) {
+        // SCSP::initialize: f = w rho0 - 1.5 w (e.F)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            double ef = 0.0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (L::e[q][d] == 1) ef += force[d];
+                else if (L::e[q][d] == -1) ef += -force[d];
+            }
+            f[q] = p.idist[q];
+            f[q] -= 1.5 * L::w[q] * ef;
+        }
+    }
+
+    double rho, u[D];
+    if (kind & KIND_ZOUHE) {
+        // PB/VB: density and velocity come from the boundary, not from
+        // calcMacroVar; at t = 0 they are initialize's rho0 and 0.
+        if (INIT) {
+            rho = p.dens0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) u[d] = 0.0;
+        } else {
+            zouhe_f64<Q>(f, zh[dsc >> DESC_LABEL_SHIFT], rho, u);
+        }
+    } else {
+        // calcMacroVar: rho = sum_q f_q (q ascending); u = (sum +-f) / rho0
+        rho = f[0];
+#pragma unroll
+        for (int q = 1; q < Q; ++q) rho += f[q];
+        if (!isfinite(rho) || rho <= 0.0) raise_status(status, 0, t);
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            double s = 0;
+#pragma unroll
+            for (int q = 1; q < Q; ++q) {
+                if (L::e[q][d] == 1) s += f[q];
+                else if (L::e[q][d] == -1) s -= f[q];
+            }
+            if (p.dens0 != 1.0) s /= p.dens0;   // x / 1 is x
+            u[d] = s;
+        }
+        // bodyForce: u += (F/2)/rho0 on GV sites
+        if (kind & KIND_GV) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) u[d] += lb.half_rho[d];
+        }
+    }
+    if (p.flags & F_FIELDS) {
+        rho_out[i] = rho;
+#pragma unroll
+        for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = u[d];
+    }
+    if (p.flags & F_ADJ) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = u[d];
+    }
+
+    // collision
+    double usq = 0;
+#pragma unroll
+    for (int d = 0; d < D; ++d) usq += u[d] * u[d];
+    if constexpr (!MRT) {
+        double uf = 0.0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) uf += u[d] * force[d];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            double ui = 0, ef = 0.0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (L::e[q][d] == 1) { ui += u[d]; ef += force[d]; }
+                else if (L::e[q][d] == -1) { ui += -u[d]; ef += -force[d]; }
+            }
+            const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
+            f[q] += (feq - f[q]) * p.omega;
+            // forceSource: G_q = w_q (3 (e.F - u.F) + 9 (e.u)(e.F))
+            if (forced) f[q] += p.omh * (L::w[q] * (3.0 * (ef - uf) + 9.0 * ui * ef));
+        }
+    } else {
+        double r[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            double ui = 0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                if (L::e[q][d] == 1) ui += u[d];
+                else if (L::e[q][d] == -1) ui += -u[d];
+            }
+            const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
+            r[q] = feq - f[q];
+        }
+        add_operator<Q>(A4, r, f);
+        if (forced) {
+            double uf = 0.0;
+#pragma unroll
+            for (int d = 0; d < D; ++d) uf += u[d] * force[d];
+            double src[Q];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                double eu = 0.0, ef = 0.0;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    if (L::e[q][d] == 1) { eu += u[d]; ef += force[d]; }
+                    else if (L::e[q][d] == -1) { eu += -u[d]; ef += -force[d]; }
+                }
+                src[q] = L::w[q] * (3.0 * (ef - uf) + 9.0 * eu * ef);
+            }
+            add_operator<Q>(B4, src, f);
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // FP64, reference operation order.
 //
@@ -99,8 +228,6 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
               const DevZouHe* __restrict__ zh)
 {
 #pragma clang fp contract(off)
-    using L = Lattice<Q>;
-    constexpr int D = L::D;
     using O = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
     uint32_t i, slot;
     if (!resolve<LAYOUT>(p, list, i, slot)) return;
@@ -126,120 +253,7 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
         for (int q = 1; q < Q; ++q) f[q] = ld(fin, off[q]);
     }
     if (fluid) {
-        const double force[3] = {lb->force[0], lb->force[1], D == 3 ? lb->force[2] : 0.0};
-        const bool forced = kind & KIND_FORCED;
-        if (INIT) {
-            // SCSP::initialize: f = w rho0 - 1.5 w (e.F)
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double ef = 0.0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    if (L::e[q][d] == 1) ef += force[d];
-                    else if (L::e[q][d] == -1) ef += -force[d];
-                }
-                f[q] = p.idist[q];
-                f[q] -= 1.5 * L::w[q] * ef;
-            }
-        }
-
-        double rho, u[D];
-        if (kind & KIND_ZOUHE) {
-            // PB/VB: density and velocity come from the boundary, not from
-            // calcMacroVar; at t = 0 they are initialize's rho0 and 0.
-            if (INIT) {
-                rho = p.dens0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) u[d] = 0.0;
-            } else {
-                zouhe_f64<Q>(f, zh[dsc >> DESC_LABEL_SHIFT], rho, u);
-            }
-        } else {
-            // calcMacroVar: rho = sum_q f_q (q ascending); u = (sum +-f) / rho0
-            rho = f[0];
-#pragma unroll
-            for (int q = 1; q < Q; ++q) rho += f[q];
-            if (!isfinite(rho) || rho <= 0.0) raise_status(status, 0, p.t);
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                double s = 0;
-#pragma unroll
-                for (int q = 1; q < Q; ++q) {
-                    if (L::e[q][d] == 1) s += f[q];
-                    else if (L::e[q][d] == -1) s -= f[q];
-                }
-                if (p.dens0 != 1.0) s /= p.dens0;   // x / 1 is x
-                u[d] = s;
-            }
-            // bodyForce: u += (F/2)/rho0 on GV sites
-            if (kind & KIND_GV) {
-#pragma unroll
-                for (int d = 0; d < D; ++d) u[d] += lb->half_rho[d];
-            }
-        }
-        if (p.flags & F_FIELDS) {
-            rho_out[i] = rho;
-#pragma unroll
-            for (int d = 0; d < D; ++d) u_out[uint64_t(d) * p.g.N + i] = u[d];
-        }
-        if (p.flags & F_ADJ) {
-#pragma unroll
-            for (int d = 0; d < D; ++d) uadj[uint64_t(d) * p.g.N + i] = u[d];
-        }
-
-        // collision
-        double usq = 0;
-#pragma unroll
-        for (int d = 0; d < D; ++d) usq += u[d] * u[d];
-        if constexpr (!MRT) {
-            double uf = 0.0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) uf += u[d] * force[d];
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double ui = 0, ef = 0.0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    if (L::e[q][d] == 1) { ui += u[d]; ef += force[d]; }
-                    else if (L::e[q][d] == -1) { ui += -u[d]; ef += -force[d]; }
-                }
-                const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
-                f[q] += (feq - f[q]) * p.omega;
-                // forceSource: G_q = w_q (3 (e.F - u.F) + 9 (e.u)(e.F))
-                if (forced) f[q] += p.omh * (L::w[q] * (3.0 * (ef - uf) + 9.0 * ui * ef));
-            }
-        } else {
-            double r[Q];
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                double ui = 0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    if (L::e[q][d] == 1) ui += u[d];
-                    else if (L::e[q][d] == -1) ui += -u[d];
-                }
-                const double feq = L::w[q] * (rho + p.dens0 * (C1 * ui + C2 * ui * ui - C3 * usq));
-                r[q] = feq - f[q];
-            }
-            add_operator<Q>(A4, r, f);
-            if (forced) {
-                double uf = 0.0;
-#pragma unroll
-                for (int d = 0; d < D; ++d) uf += u[d] * force[d];
-                double src[Q];
-#pragma unroll
-                for (int q = 0; q < Q; ++q) {
-                    double eu = 0.0, ef = 0.0;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        if (L::e[q][d] == 1) { eu += u[d]; ef += force[d]; }
-                        else if (L::e[q][d] == -1) { eu += -u[d]; ef += -force[d]; }
-                    }
-                    src[q] = L::w[q] * (3.0 * (ef - uf) + 9.0 * eu * ef);
-                }
-                add_operator<Q>(B4, src, f);
-            }
-        }
+        scsp_site_f64<Q, MRT, INIT>(p, *lb, dsc, i, p.t, A4, B4, rho_out, u_out, uadj, status, zh, f);
     }
     double chk = 0.0;   // stays 0 while every population is finite
 #pragma unroll
@@ -248,6 +262,70 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
         st(fout, pop_index<Q, BLK, O>(P, q, slot), f[q]);
     }
     if (!(chk == 0.0)) raise_status(status, 4, p.t);
+}
+
+// ---------------------------------------------------------------------------
+// Several FP64 steps of a dense lattice of few sites (scsp_few_sites), one workgroup,
+// one site per thread, the populations in LDS between steps.  A launch per step
+// costs 5 us whatever the lattice; here a step costs its arithmetic, two
+// barriers and the LDS round trip.  The sites' links and pull sources are
+// resolved once per launch.  Per step, launch per step -> here: D2Q9 MRT 320
+// sites 4.9 -> 2.3 us, 1023 sites 4.7 -> 4.3 (SRT 3.8 -> 2.3); D3Q19 MRT 256
+// sites 9.1 -> 4.6, 512 sites 9.1 -> 7.7 (SRT 4.7 -> 2.3).  Bound by the FP64
+// issue of the one CU, so larger lattices take a launch per step.
+// ---------------------------------------------------------------------------
+template <int Q, bool MRT, int LAYOUT>
+__global__ void __launch_bounds__(scsp_few_sites(Q))
+scsp_steps_f64(ScspParams p, uint32_t steps, const double* fin, double* fout, const uint32_t* __restrict__ desc,
+               const DevLabel* __restrict__ lab, const double* __restrict__ A4, const double* __restrict__ B4,
+               DevStatus* __restrict__ status, const DevZouHe* __restrict__ zh)
+{
+#pragma clang fp contract(off)
+    constexpr uint32_t FEW_SITES = scsp_few_sites(Q);
+    __shared__ double pop[Q * FEW_SITES];
+    const uint32_t i = threadIdx.x, N = uint32_t(p.g.N);
+    bool active = i < N, fluid = false;
+    uint32_t dsc = 0, off[Q];
+    DevLabel lb{};
+    double f[Q];
+    if (active) {
+        dsc = desc[i];
+        lb = lab[dsc >> DESC_LABEL_SHIFT];
+        fluid = lb.kind & KIND_FLUID;
+        active = fluid || LAYOUT == DENSE_ALL;
+    }
+    if (active) {
+        pull_offsets<Q, LAYOUT, uint32_t>(nullptr, dsc, i, make_stencil(p.g, i), p.g.nx, FEW_SITES, off);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            f[q] = fin[size_t(q) * N + i];
+            pop[q * FEW_SITES + i] = f[q];
+        }
+    }
+#pragma unroll 1
+    for (uint32_t k = 0; k < steps; ++k) {
+        __syncthreads();
+        if (active) {
+            f[0] = pop[i];
+#pragma unroll
+            for (int q = 1; q < Q; ++q) f[q] = pop[off[q]];
+        }
+        __syncthreads();
+        if (fluid)
+            scsp_site_f64<Q, MRT, false>(p, lb, dsc, i, p.t + k, A4, B4, nullptr, nullptr, nullptr, status, zh, f);
+        if (active) {
+            double chk = 0.0;   // stays 0 while every population is finite
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                chk = __builtin_fma(f[q], 0.0, chk);
+                pop[q * FEW_SITES + i] = f[q];
+            }
+            if (!(chk == 0.0)) raise_status(status, 4, p.t + k);
+        }
+    }
+    if (active)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) fout[size_t(q) * N + i] = f[q];
 }
 
 // ---------------------------------------------------------------------------
@@ -378,6 +456,30 @@ hipError_t launch_scsp(int Q, bool mrt, bool init, bool fp32, int layout, const 
         else init ? launch_scsp_q<9, false, true>(p, b, fp32, layout, s)
                   : launch_scsp_q<9, false, false>(p, b, fp32, layout, s);
     }
+    return hipGetLastError();
+}
+
+template <int Q, bool MRT>
+static void launch_scsp_steps_q(const ScspParams& p, const ScspBuffers& b, bool all, uint32_t steps, hipStream_t s)
+{
+    const dim3 block((uint32_t(p.g.N) + 63u) / 64u * 64u);
+    const double* fin = static_cast<const double*>(b.fin);
+    double* fout = static_cast<double*>(b.fout);
+    if (all)
+        hipLaunchKernelGGL((scsp_steps_f64<Q, MRT, DENSE_ALL>), dim3(1), block, 0, s, p, steps, fin, fout, b.desc,
+                           b.lab, b.A4, b.B4, b.status, b.zh);
+    else
+        hipLaunchKernelGGL((scsp_steps_f64<Q, MRT, DENSE_FLUID>), dim3(1), block, 0, s, p, steps, fin, fout, b.desc,
+                           b.lab, b.A4, b.B4, b.status, b.zh);
+}
+
+hipError_t launch_scsp_steps(int Q, bool mrt, int layout, uint32_t steps, const ScspParams& p, const ScspBuffers& b,
+                             hipStream_t s)
+{
+    if (p.g.N == 0 || p.g.N > scsp_few_sites(Q) || layout == SPARSE || (p.flags & (F_FIELDS | F_ADJ))) return hipErrorInvalidValue;
+    const bool all = layout == DENSE_ALL;
+    if (Q == 19) mrt ? launch_scsp_steps_q<19, true>(p, b, all, steps, s) : launch_scsp_steps_q<19, false>(p, b, all, steps, s);
+    else mrt ? launch_scsp_steps_q<9, true>(p, b, all, steps, s) : launch_scsp_steps_q<9, false>(p, b, all, steps, s);
     return hipGetLastError();
 }
 
