@@ -22,6 +22,7 @@
 #include "setup.h"
 
 namespace lbf {
+hipError_t launch_color_steps(int Q, bool mrt, bool stream_solids, uint32_t steps, const ColorArgs& a, hipStream_t s);
 hipError_t launch_scsp_steps(int Q, bool mrt, int layout, uint32_t steps, const ScspParams& p, const ScspBuffers& b,
                              hipStream_t s);
 hipError_t launch_scsp(int Q, bool mrt, bool init, bool fp32, int layout, const ScspParams& p,
@@ -817,20 +818,38 @@ static int run_step(lbf_ctx* c, bool init, uint32_t flags)
     return 0;
 }
 
-// n plain steps.  Small FP64 single-phase lattices take several per launch; the
+// n plain steps.  Small FP64 lattices take several per launch; the
 // chunk bounds a launch's length (a few ms).  The populations end in the
 // buffer in which single steps would leave them.
 static int advance_steps(lbf_ctx* c, uint64_t n)
 {
     constexpr uint64_t CHUNK = 512;
-    if (c->NP == 1 && c->elem == 8 && c->layout != 2 && c->N > 0 && c->N <= scsp_few_sites(c->Q)) {
+    const bool mrt = c->d.equil == LBF_MRT, solids = c->d.flags & LBF_STREAM_SOLIDS;
+    bool many = false;
+    ColorArgs a{};
+    if (c->NP == 1) {
+        many = c->elem == 8 && c->layout != 2 && c->N > 0 && c->N <= scsp_few_sites(c->Q);
+    } else if (c->elem == 8) {
+        a = color_args(c, 0u);
+        const uint32_t items = std::max(a.nfitems, solids ? a.nitems : 0u);
+        many = a.plain && !a.csf && !a.tanh_wall && items > 0 && items <= color_few_items(c->Q);
+    }
+    if (many) {
         while (n > 1) {
             const uint32_t steps = uint32_t(std::min(n, CHUNK));
-            ScspParams p = scsp_params(c, 0u);
-            p.t = c->t + 1;
-            ScspBuffers b = scsp_buffers(c, false);
-            if (steps % 2 == 0) b.fout = c->f[c->cur];
-            const hipError_t e = launch_scsp_steps(c->Q, c->d.equil == LBF_MRT, c->layout, steps, p, b, c->stream);
+            hipError_t e;
+            if (c->NP == 1) {
+                ScspParams p = scsp_params(c, 0u);
+                p.t = c->t + 1;
+                ScspBuffers b = scsp_buffers(c, false);
+                if (steps % 2 == 0) b.fout = c->f[c->cur];
+                e = launch_scsp_steps(c->Q, mrt, c->layout, steps, p, b, c->stream);
+            } else {
+                a.t = c->t + 1;
+                a.fin = static_cast<const double*>(c->f[c->cur]);
+                a.fout = static_cast<double*>(c->f[c->cur ^ 1]);
+                e = launch_color_steps(c->Q, mrt, solids, steps, a, c->stream);
+            }
             if (e != hipSuccess) return fail(c, std::string("HIP error: kernel launch: ") + hipGetErrorString(e));
             c->cur ^= int(steps % 2);
             c->t += steps;

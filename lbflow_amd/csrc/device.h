@@ -190,6 +190,10 @@ struct ScspBuffers {
     const DevZouHe* zh;      // Zou-He boundary per label
 };
 
+// Colour lattices up to this many items of their work orders likewise (at the
+// limits both ways take the same time).
+constexpr uint32_t color_few_items(int Q) { return Q == 9 ? 768u : 512u; }
+
 struct ColorArgs {
     GridDev g;
     const double* fin;       // [phase][q][site]

@@ -1,5 +1,5 @@
 """Lattices whose FP64 steps run several to a launch: advance(n) equals n single
-steps bit for bit, populations and report history alike, for sizes up to and
+steps bit for bit in both models, for sizes up to and
 beyond the limit, rows of one site, no solid and hardly any fluid, an odd and
 an even number of steps and more than one launch; and a failure is recorded at
 the step at which single steps record it."""
@@ -21,6 +21,29 @@ def _spec(shape, phi, eq):
 def _engine(spec, solids):
     from lbflow_amd.engine import FP64, Engine
     return Engine(CS.lattice(spec), CS.geometry(spec), FP64, solids).init()
+
+
+def _colour(shape, phi, eq, harmonic):
+    rng = np.random.default_rng(sum(shape))
+    g = np.where(rng.random(shape) < phi, np.where(rng.random(shape) < 0.5, 75, 76), 255).astype(np.uint8)
+    labels = [CS.label_line(75, 'GV', 1e-5, 1, 0), CS.label_line(76, 'VD', phase=1), CS.label_line(255, 'SD', 60)]
+    kw = dict(viscosity_interpolation='harmonic', tau=(0.9, 0.6)) if harmonic else dict(tau=(1.0, 1.0))
+    return CS.make('small', g, labels, model='color', eq=eq, sigma=1e-3, beta=0.7, **kw)
+
+
+@pytest.mark.parametrize('shape,phi,eq,solids,harmonic', [
+    ((1, 9, 7), 0.6, 'MRT', True, False), ((1, 24, 32), 1.0, 'MRT', True, True), ((1, 31, 24), 0.8, 'SRT', True, True),
+    ((1, 32, 32), 0.6, 'MRT', False, False), ((8, 8, 8), 0.7, 'MRT', True, True), ((8, 8, 8), 1.0, 'SRT', False, False),
+    ((8, 8, 9), 0.4, 'MRT', False, False), ((4, 4, 4), 0.0, 'MRT', True, False)])
+def test_colour_advance_equals_single_steps(shape, phi, eq, solids, harmonic):
+    spec = _colour(shape, phi, eq, harmonic)
+    a, b = _engine(spec, solids), _engine(spec, solids)
+    for n in (1, 2, 7, 40):
+        a.advance(n)
+        for _ in range(n):
+            b.step(0)
+        assert a.t == b.t and a.status()[0] == b.status()[0]
+        assert np.array_equal(a.populations().view(np.uint64), b.populations().view(np.uint64))
 
 
 @pytest.mark.parametrize('shape,phi,eq,solids', [
