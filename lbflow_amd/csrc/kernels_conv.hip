@@ -572,6 +572,97 @@ conv_fwd_rows(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restric
 }
 
 // ---------------------------------------------------------------------------
+// forward, 3x3x3 from 8 channels (the input layer), BF16 output, sides from 16,
+// 32 output channels: a workgroup's 16 x 8 x 8 voxels and their one-voxel
+// periodic halo lie in LDS (16 bytes a voxel), all the weights in registers.  A
+// k step of the direct kernel is 4 taps; lane group grp reads tap 4 s + grp of
+// its 16 consecutive voxels, 256 consecutive bytes.  Operands and weight rows
+// are arranged as in the rows kernel, 16 bytes a store.  Bound by the stores:
+// 8 x 64^3 102 -> 43 us (151 MB, 3.5 TB/s), where the direct kernel gathers
+// every tap of every voxel through L1.
+// ---------------------------------------------------------------------------
+template <int ACT, bool BIAS>
+__global__ void __launch_bounds__(256)
+conv_fwd_input(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restrict__ w,
+               const float* __restrict__ bias, __bf16* __restrict__ out)
+{
+    constexpr int KP = conv_kp(8, 27), STEPS = KP / 32;
+    constexpr int HX = 18, HY = 10, HV = HX * HY * 10, TRIPS = (HV + 255) / 256;
+    static_assert(KP == 224, "27 taps of 8 channels and one of zeros");
+    __shared__ __attribute__((aligned(16))) __bf16 tile[HV * 8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r16 = lane & 15, grp = lane >> 4;
+    const uint32_t ls = g.log_s, m = (1u << ls) - 1u;
+    // block -> sample and origin
+    const uint32_t lx = ls - 4, ly = ls - 3, b = blockIdx.x & ((1u << (lx + 2 * ly)) - 1u);
+    const uint32_t smp = blockIdx.x >> (lx + 2 * ly);
+    const uint32_t x0 = (b & ((1u << lx) - 1u)) << 4, y0 = ((b >> lx) & ((1u << ly) - 1u)) << 3,
+                   z0 = (b >> (lx + ly)) << 3;
+    const size_t sbase = size_t(smp) << (3 * ls);
+    {
+        bf16x8 r[TRIPS];
+#pragma unroll
+        for (int t = 0; t < TRIPS; ++t) {
+            const int v = int(threadIdx.x) + 256 * t;
+            const int hz = v / (HX * HY), hy = v / HX % HY, hx = v % HX;
+            const uint32_t x = (x0 + uint32_t(hx) - 1u) & m, y = (y0 + uint32_t(hy) - 1u) & m,
+                           z = (z0 + uint32_t(hz) - 1u) & m;
+            // threads past the halo's end read a voxel of the sample and store nothing
+            r[t] = *reinterpret_cast<const bf16x8*>(in + (sbase + ((z << (2 * ls)) | (y << ls) | x)) * g.in_stride);
+        }
+#pragma unroll
+        for (int t = 0; t < TRIPS; ++t) {
+            const int v = int(threadIdx.x) + 256 * t;
+            if (v < HV) *reinterpret_cast<bf16x8*>(tile + v * 8) = r[t];
+        }
+    }
+    // weight row r16 of tile j is output channel 8 (r16 / 4) + 4 j + r16 % 4: a
+    // lane's results are then channels 8 grp .. 8 grp + 7
+    bf16x8 wf[STEPS][2];
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+            wf[s][j] = *reinterpret_cast<const bf16x8*>(w + size_t(8 * (r16 >> 2) + 4 * j + (r16 & 3)) * KP + 32 * s + 8 * grp);
+    float bs[8];
+    if constexpr (BIAS)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) bs[e] = bias[8 * grp + e];
+    int off[STEPS];   // this lane's tap of each step, from the row's first halo voxel
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+        const int tap = 4 * s + grp < 27 ? 4 * s + grp : 26;   // (the 28th multiplies zeros)
+        off[s] = ((tap / 9 * HY + tap / 3 % 3) * HX + tap % 3 + r16) * 8;
+    }
+    __syncthreads();
+    // the wave's 16 rows: z layers 2 wave and 2 wave + 1, 8 rows each
+#pragma unroll 2
+    for (int row = 0; row < 16; ++row) {
+        const int lz = 2 * wave + (row >> 3), lyv = row & 7;
+        const __bf16* base = tile + (lz * HY + lyv) * HX * 8;
+        f32x4 acc[2] = {f32x4{0.0f, 0.0f, 0.0f, 0.0f}, f32x4{0.0f, 0.0f, 0.0f, 0.0f}};
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            bf16x8 a = *reinterpret_cast<const bf16x8*>(base + off[s]);
+            if (4 * s + 3 >= 27 && grp == 3) a = bf16_zero();
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[s][j], a, acc[j], 0, 0, 0);
+        }
+        const size_t v = sbase + ((size_t(z0 + lz) << (2 * ls)) | (size_t(y0 + lyv) << ls) | (x0 + r16));
+        bf16x8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            float r = acc[e >> 2][e & 3];
+            if constexpr (BIAS) r += bs[e];
+            if (ACT == ACT_RELU) r = r > 0.0f ? r : 0.0f;
+            o[e] = __bf16(r);
+        }
+        *reinterpret_cast<bf16x8*>(out + v * g.out_stride + 8 * grp) = o;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // forward (and input gradient), 3x3x3 with Cin a multiple of 32, sides below 8
 // (the coarse levels of small volumes): a few dozen voxels against up to 3.5 MB
 // of weights.  One wave per 16 output channels and MT tiles of 16 voxels, in
@@ -1332,6 +1423,16 @@ struct ConvLaunch {
                 hipLaunchKernelGGL((conv_fwd_coarse<CIN, COUT, 4, ACT, BIAS, OUTF32>),
                                    dim3((g.nvox + 63u) / 64u, COUT / 16), dim3(64), 0, s, g, in, w, bias, out);
         } else {
+            // The input layer with whole 16-byte rows, where a block of 16 x 8 x 8
+            // voxels fits a sample.
+            if constexpr (CIN == 8 && COUT == 32 && TAPS == 27 && !OUTF32 && ACT != ACT_RELU_GATE) {
+                const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out);
+                if (g.log_s >= 4 && at % 16 == 0 && (g.in_stride | g.out_stride) % 8 == 0) {
+                    hipLaunchKernelGGL((conv_fwd_input<ACT, BIAS>), dim3(g.nvox / 1024u), dim3(256), 0, s, g, in, w, bias,
+                                       static_cast<__bf16*>(out));
+                    return;
+                }
+            }
             const dim3 grid((g.nvox + 255u) / 256u, (COUT + BN_FWD - 1) / BN_FWD);
             hipLaunchKernelGGL((conv_fwd<CIN, COUT, TAPS, BN_FWD, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g, in, w,
                                bias, out);

@@ -269,10 +269,11 @@ scsp_step_f64(ScspParams p, const double* __restrict__ fin, double* __restrict__
 // one site per thread, the populations in LDS between steps.  A launch per step
 // costs 5 us whatever the lattice; here a step costs its arithmetic, two
 // barriers and the LDS round trip.  The sites' links and pull sources are
-// resolved once per launch.  Per step, launch per step -> here: D2Q9 MRT 320
-// sites 4.9 -> 2.3 us, 1023 sites 4.7 -> 4.3 (SRT 3.8 -> 2.3); D3Q19 MRT 256
-// sites 9.1 -> 4.6, 512 sites 9.1 -> 7.7 (SRT 4.7 -> 2.3).  Bound by the FP64
-// issue of the one CU, so larger lattices take a launch per step.
+// resolved once per launch.  Per step, launch per step -> here: D2Q9 320 sites
+// MRT 4.3 -> 2.3 us, SRT 4.1 -> 1.2, 1023 sites MRT 4.7 -> 4.3, SRT 4.0 -> 2.3;
+// D3Q19 256 sites MRT 8.7 -> 4.6, SRT 4.4 -> 1.6, 512 sites MRT 9.1 -> 7.7, SRT
+// 4.7 -> 2.3.  Bound by the FP64 issue of the one CU, so larger lattices take a
+// launch per step.
 // ---------------------------------------------------------------------------
 template <int Q, bool MRT, int LAYOUT>
 __global__ void __launch_bounds__(scsp_few_sites(Q))
