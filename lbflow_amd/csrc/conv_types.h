@@ -28,6 +28,7 @@ struct ConvGeom {
     float* kpart;            // forward split over input channels: FP32 partials [split][voxel][Cout]
                              // (null: no split)
     uint32_t kpart_floats;   // floats available at kpart
+    uint32_t out_channels;   // 1x1x1 head: store only this many output channels (0: all)
 };
 
 // ACT_RELU_GATE: out = gate > 0 ? x : 0, the ReLU gradient of the layer

@@ -147,7 +147,7 @@ conv_fwd(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restrict__ w
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
         const int co = co0 + 16 * j + r16;
-        if (co >= COUT) continue;
+        if (co >= COUT || (TAPS == 1 && g.out_channels && uint32_t(co) >= g.out_channels)) continue;
         const float bb = BIAS ? bias[co] : 0.0f;
 #pragma unroll
         for (int i = 0; i < 4; ++i)

@@ -53,18 +53,21 @@ __global__ void net_input(const uint8_t* __restrict__ mask, uint32_t nvox, __bf1
     st8(Chan{x0, 8, 0}, v, 0, x);
 }
 
-// out[V][c] = mean of the 8 children of V.  ls = log2 side of the output.
+// out[V][c] = mean of the 8 children of V, their 8 loads in flight together.
+// ls = log2 side of the output.
 __global__ void net_pool(Chan in, Chan out, uint32_t C, uint32_t ls, uint32_t nvox_out)
 {
     const uint32_t t = blockIdx.x * 256u + threadIdx.x;
     const uint32_t V = t / (C / 8), c = (t % (C / 8)) * 8;
     if (V >= nvox_out) return;
     float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int j = 0; j < 8; ++j) {
-        const bf16x8 a = ld8(in, child_of(V, ls, j), c);
+    bf16x8 a[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s[k] += float(a[k]);
-    }
+    for (int j = 0; j < 8; ++j) a[j] = ld8(in, child_of(V, ls, j), c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[k] += float(a[j][k]);
 #pragma unroll
     for (int k = 0; k < 8; ++k) s[k] *= 0.125f;
     st8(out, V, c, s);
@@ -247,14 +250,6 @@ net_adam(float* __restrict__ p, float* __restrict__ m, float* __restrict__ v, co
     if (pb) pb[i] = __bf16(pi);
 }
 
-// out4[v][c] = out16[v][c], c < 4 (the head's real channels).
-__global__ void net_head4(const float* __restrict__ out16, uint32_t nvox, float* __restrict__ out4)
-{
-    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-    if (i >= nvox * 4u) return;
-    out4[i] = out16[size_t(i >> 2) * 16 + (i & 3u)];
-}
-
 // Physical fields of a prediction: out4[v][c] = out16[v][c] scale[c] +
 // offset[c], the velocity channels (c < 3) zero where mask[v] is 0 (solid).
 __global__ void net_head_fields(const float* __restrict__ out16, const uint8_t* __restrict__ mask, uint32_t nvox,
@@ -360,11 +355,6 @@ hipError_t launch_net_adam(float* p, float* m, float* v, const float* g, uint32_
                            float eps, float c1, float c2, __bf16* pb, hipStream_t s)
 {
     hipLaunchKernelGGL(net_adam, grid_for(n), dim3(256), 0, s, p, m, v, g, n, lr, b1, b2, eps, c1, c2, pb);
-    return hipGetLastError();
-}
-hipError_t launch_net_head4(const float* out16, uint32_t nvox, float* out4, hipStream_t s)
-{
-    hipLaunchKernelGGL(net_head4, grid_for(uint64_t(nvox) * 4), dim3(256), 0, s, out16, nvox, out4);
     return hipGetLastError();
 }
 hipError_t launch_net_head_fields(const float* out16, const uint8_t* mask, uint32_t nvox, const float* scale,
