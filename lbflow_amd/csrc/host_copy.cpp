@@ -22,7 +22,8 @@ constexpr size_t SMALL = size_t(8) << 20;
 
 class HostStage {
   public:
-    int device = 0;
+    explicit HostStage(int dev) : device(dev) {}
+    const int device;
     std::mutex busy;   // one copy at a time uses the buffers
     char* pinned = nullptr;
     hipEvent_t done[WORKERS][2] = {};
@@ -34,7 +35,7 @@ class HostStage {
                 if (e) (void)hipEventDestroy(e);
         if (pinned) (void)hipHostFree(pinned);
     }
-    // busy held
+    // busy held, the stage's device current
     bool ready()
     {
         if (pinned) return true;
@@ -53,22 +54,43 @@ class HostStage {
     char* buffer(unsigned w, int k) { return pinned + (size_t(w) * 2 + size_t(k)) * CHUNK; }
 };
 
-std::shared_ptr<HostStage> host_stage()
+static std::shared_ptr<HostStage> host_stage(int dev)
 {
     static std::mutex lock;
     static std::map<int, std::weak_ptr<HostStage>> stages;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     std::lock_guard<std::mutex> hold(lock);
     std::shared_ptr<HostStage> s = stages[dev].lock();
-    if (!s) {
-        s = std::make_shared<HostStage>();
-        s->device = dev;
-        stages[dev] = s;
-    }
+    if (!s) stages[dev] = s = std::make_shared<HostStage>(dev);
     return s;
 }
 
+namespace {
+// Makes a device the calling thread's current one for a scope: events belong to
+// the device that is current when they are created, and the caller's choice
+// stays the caller's.
+class CurrentDevice {
+  public:
+    explicit CurrentDevice(int dev)
+    {
+        if (hipGetDevice(&before) != hipSuccess) return;
+        set = before == dev || hipSetDevice(dev) == hipSuccess;
+        changed = set && before != dev;
+    }
+    ~CurrentDevice()
+    {
+        if (changed) (void)hipSetDevice(before);
+    }
+    CurrentDevice(const CurrentDevice&) = delete;
+    CurrentDevice& operator=(const CurrentDevice&) = delete;
+    bool set = false;
+
+  private:
+    int before = 0;
+    bool changed = false;
+};
+}  // namespace
+
+// The stage's device is current.
 static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_t bytes, hipStream_t s)
 {
     const size_t chunks = (bytes + CHUNK - 1) / CHUNK;
@@ -77,7 +99,7 @@ static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_
     auto work = [&](unsigned w) {
         constexpr size_t NONE = ~size_t(0);
         size_t held[2] = {NONE, NONE};
-        if (hipSetDevice(st.device) != hipSuccess) error = int(hipErrorInvalidDevice);
+        if (w && hipSetDevice(st.device) != hipSuccess) error = int(hipErrorInvalidDevice);   // 0: the caller's thread
         for (int cur = 0;; cur ^= 1) {
             hipError_t e = hipSuccess;
             const size_t k = error == int(hipSuccess) ? next++ : chunks;
@@ -115,10 +137,12 @@ static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_
 
 hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void* src, size_t bytes, hipStream_t s)
 {
-    if (bytes >= SMALL) {
+    hipDevice_t dev = 0;
+    if (bytes >= SMALL && hipStreamGetDevice(s, &dev) == hipSuccess) {
         try {
-            if (!stage) stage = host_stage();
-            if (stage) {
+            const CurrentDevice current(dev);
+            if (!stage) stage = host_stage(dev);
+            if (current.set) {
                 std::lock_guard<std::mutex> hold(stage->busy);
                 if (stage->ready())
                     return copy_parallel(*stage, static_cast<char*>(dst), static_cast<const char*>(src), bytes, s);

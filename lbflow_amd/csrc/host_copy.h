@@ -17,11 +17,12 @@ namespace lbf {
 // The pinned buffers and events of one GPU (32 MiB), shared by every object
 // of the process that holds one and released with the last of them.
 class HostStage;
-std::shared_ptr<HostStage> host_stage();
 
 // Copies `bytes` from device memory to dst, ordered after the work queued on
-// s, and returns when dst is complete.  `stage` is the caller's handle, taken
-// on the first large copy and kept.  Any number of threads may copy at once.
+// s (a created stream), and returns when dst is complete.  Works on the
+// stream's device, whichever is current.  `stage` is the caller's handle for
+// that device, taken on the first large copy and kept; any number of threads,
+// each with its own handle, may copy at once.
 hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void* src, size_t bytes, hipStream_t s);
 
 }  // namespace lbf

@@ -1,0 +1,69 @@
+// One scenario of csrc/host_copy.cpp on the stand-in runtime of hip/hip_runtime.h;
+// exit status 0 if it holds.  Every wrong result prints a line.
+#include "host_copy.h"
+
+#include <cstdio>
+#include <cstdint>
+#include <new>
+#include <vector>
+#include <string>
+
+// The allocation that fails: the n-th of the main thread from now on (negative: none).
+static thread_local int news_left = -1;
+void* operator new(size_t n)
+{
+    if (news_left >= 0 && news_left-- == 0) throw std::bad_alloc();
+    if (void* p = std::malloc(n)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+static int wrong = 0;
+static void check(bool ok, const char* what)
+{
+    if (ok) return;
+    std::printf("wrong: %s\n", what);
+    ++wrong;
+}
+
+struct Data {
+    std::vector<char> src, dst;
+    explicit Data(size_t n) : src(n), dst(n, 0)
+    {
+        for (size_t i = 0; i < n; ++i) src[i] = char(i * 2654435761u >> 13);
+    }
+    bool arrived() const { return src == dst; }
+};
+
+static hipError_t copy(std::shared_ptr<lbf::HostStage>& stage, Data& d, hipStream_t s)
+{
+    return lbf::copy_to_host(stage, d.dst.data(), d.src.data(), d.src.size(), s);
+}
+
+// A copy on a stream of another device than the caller's current one, as the first copy on
+// that device and as a later one.
+static void other_device()
+{
+    FakeStream s;
+    s.device = 1;
+    std::shared_ptr<lbf::HostStage> first, later;
+    for (int current : {0, 1, 0}) {
+        for (auto* stage : {&first, &later}) {
+            Data d((size_t(20) << 20) + 12345);
+            fake::current = current;
+            check(copy(*stage, d, &s) == hipSuccess, "the copy succeeds");
+            check(d.arrived(), "the data arrive");
+            check(fake::current == current, "the caller's device is still current");
+        }
+    }
+    check(first == later && first, "one stage serves the device");
+}
+
+int main(int argc, char** argv)
+{
+    const std::string name = argc > 1 ? argv[1] : "";
+    if (name == "other_device") other_device();
+    else check(false, "unknown scenario");
+    return wrong != 0;
+}
