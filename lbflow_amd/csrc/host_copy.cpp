@@ -4,9 +4,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -127,8 +127,10 @@ static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_
     pool.reserve(n);
     try {
         for (unsigned w = 1; w < n; ++w) pool.emplace_back(work, w);
-    } catch (const std::system_error&) {
-        // the threads that did start and this one take all chunks
+    } catch (const std::exception&) {
+        // no thread or no memory for one: those that did start and this one take all
+        // chunks (and are joined: a std::thread that goes out of scope unjoined
+        // ends the process)
     }
     work(0);
     for (std::thread& t : pool) t.join();

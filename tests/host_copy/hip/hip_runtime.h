@@ -7,7 +7,6 @@
 #include <cstddef>
 #include <cstdlib>
 #include <cstring>
-#include <functional>
 #include <mutex>
 #include <vector>
 
@@ -21,14 +20,20 @@ struct hipPointerAttribute_t {
     hipMemoryType type;
     int device;
 };
+struct FakeCopy {
+    void* dst;
+    const void* src;
+    size_t n;
+};
 struct FakeStream {
     int device = 0;
     std::mutex lock;
-    std::vector<std::function<void()>> queued;
+    std::vector<FakeCopy> queued;
+    FakeStream() { queued.reserve(1024); }   // (the runtime's calls throw nothing)
 };
 struct FakeEvent {
-    int device = 0;
-    FakeStream* on = nullptr;
+    int device;
+    FakeStream* on;
 };
 typedef FakeStream* hipStream_t;
 typedef FakeEvent* hipEvent_t;
@@ -48,7 +53,7 @@ inline bool spent(std::atomic<int>& left) { return left >= 0 && left-- == 0; }
 inline void drain(FakeStream* s)
 {
     std::lock_guard<std::mutex> hold(s->lock);
-    for (auto& f : s->queued) f();
+    for (auto& c : s->queued) std::memcpy(c.dst, c.src, c.n);
     s->queued.clear();
 }
 inline size_t pending(FakeStream* s)
@@ -80,13 +85,15 @@ inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned)
         fake::event_creations_left = 0;
         return hipErrorOutOfMemory;
     }
-    *e = new FakeEvent{fake::current, nullptr};
+    *e = static_cast<FakeEvent*>(std::malloc(sizeof(FakeEvent)));
+    (*e)->device = fake::current;
+    (*e)->on = nullptr;
     ++fake::events;
     return hipSuccess;
 }
 inline hipError_t hipEventDestroy(hipEvent_t e)
 {
-    delete e;
+    std::free(e);
     --fake::events;
     return hipSuccess;
 }
@@ -111,7 +118,7 @@ inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpy
 {
     ++fake::staged;
     std::lock_guard<std::mutex> hold(s->lock);
-    s->queued.push_back([=] { std::memcpy(dst, src, n); });
+    s->queued.push_back(FakeCopy{dst, src, n});
     return hipSuccess;
 }
 inline hipError_t hipMemcpyWithStream(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t s)

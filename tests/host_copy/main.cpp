@@ -60,10 +60,26 @@ static void other_device()
     check(first == later && first, "one stage serves the device");
 }
 
+// An allocation of the calling thread fails, each one of the copy's in turn: while the
+// handle is taken, between the threads that start, after them.
+static void no_memory()
+{
+    FakeStream s;
+    for (int n = 0; n < 16; ++n) {
+        std::shared_ptr<lbf::HostStage> stage;
+        Data d((size_t(40) << 20) + 1);
+        news_left = n;
+        const hipError_t e = copy(stage, d, &s);
+        news_left = -1;
+        check(e == hipSuccess && d.arrived(), "the data arrive");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "other_device") other_device();
+    else if (name == "no_memory") no_memory();
     else check(false, "unknown scenario");
     return wrong != 0;
 }
