@@ -28,13 +28,7 @@ class HostStage {
     char* pinned = nullptr;
     hipEvent_t done[WORKERS][2] = {};
 
-    ~HostStage()
-    {
-        for (auto& w : done)
-            for (hipEvent_t e : w)
-                if (e) (void)hipEventDestroy(e);
-        if (pinned) (void)hipHostFree(pinned);
-    }
+    ~HostStage() { release(); }
     // busy held, the stage's device current
     bool ready()
     {
@@ -45,13 +39,25 @@ class HostStage {
         for (auto& w : done)
             for (hipEvent_t& e : w)
                 if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                    (void)hipHostFree(pinned);
-                    pinned = nullptr;
+                    e = nullptr;
+                    release();
                     return false;
                 }
         return true;
     }
     char* buffer(unsigned w, int k) { return pinned + (size_t(w) * 2 + size_t(k)) * CHUNK; }
+
+  private:
+    void release()
+    {
+        for (auto& w : done)
+            for (hipEvent_t& e : w) {
+                if (e) (void)hipEventDestroy(e);
+                e = nullptr;
+            }
+        if (pinned) (void)hipHostFree(pinned);
+        pinned = nullptr;
+    }
 };
 
 static std::shared_ptr<HostStage> host_stage(int dev)

@@ -75,11 +75,32 @@ static void no_memory()
     }
 }
 
+// The creation of an event fails: the plain copy serves, nothing made on the way stays
+// behind, and a later copy finds the stage whole.
+static void no_event()
+{
+    FakeStream s;
+    for (int n : {0, 1, 7, 15}) {
+        std::shared_ptr<lbf::HostStage> stage;
+        fake::event_creations_left = n;
+        Data d(size_t(9) << 20);
+        check(copy(stage, d, &s) == hipSuccess && d.arrived(), "the plain copy serves");
+        check(fake::events == 0 && fake::pinned == 0, "what was made is given back");
+        fake::event_creations_left = -1;
+        Data e(size_t(9) << 20);
+        check(copy(stage, e, &s) == hipSuccess && e.arrived(), "a later copy serves");
+        check(fake::events == 16 && fake::pinned == 1, "one set of events and buffers");
+        stage.reset();
+        check(fake::events == 0 && fake::pinned == 0, "released with the last handle");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "other_device") other_device();
     else if (name == "no_memory") no_memory();
+    else if (name == "no_event") no_event();
     else check(false, "unknown scenario");
     return wrong != 0;
 }
