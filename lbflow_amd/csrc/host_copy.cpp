@@ -140,6 +140,8 @@ static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_
     }
     work(0);
     for (std::thread& t : pool) t.join();
+    // a copy whose event could not be recorded is still on its way into a buffer
+    if (error != int(hipSuccess)) (void)hipStreamSynchronize(s);
     return hipError_t(error.load());
 }
 

@@ -95,12 +95,30 @@ static void no_event()
     }
 }
 
+// An event cannot be recorded behind a copy that is already queued: the call reports it
+// after that copy is done, since the next call fills the same buffers.
+static void no_record()
+{
+    FakeStream s;
+    for (int n : {0, 3, 9}) {
+        std::shared_ptr<lbf::HostStage> stage;
+        fake::records_left = n;
+        Data d((size_t(40) << 20) + 77);
+        check(copy(stage, d, &s) != hipSuccess, "the failure is reported");
+        check(fake::pending(&s) == 0, "no copy into the buffers is left in flight");
+        fake::records_left = -1;
+        Data e((size_t(40) << 20) + 77);
+        check(copy(stage, e, &s) == hipSuccess && e.arrived(), "a later copy serves");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
     if (name == "other_device") other_device();
     else if (name == "no_memory") no_memory();
     else if (name == "no_event") no_event();
+    else if (name == "no_record") no_record();
     else check(false, "unknown scenario");
     return wrong != 0;
 }
