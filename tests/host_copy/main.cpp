@@ -112,6 +112,20 @@ static void no_record()
     }
 }
 
+// Below the size from which threads help: one blocking call of the runtime.
+static void small()
+{
+    FakeStream s;
+    for (size_t n : {size_t(1), size_t(4096), (size_t(8) << 20) - 1}) {
+        std::shared_ptr<lbf::HostStage> stage;
+        fake::plain = fake::staged = 0;
+        Data d(n);
+        check(copy(stage, d, &s) == hipSuccess && d.arrived(), "the data arrive");
+        check(fake::plain == 1 && fake::staged == 0, "by one blocking call");
+        check(!stage && fake::pinned == 0, "without a stage");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
@@ -119,6 +133,7 @@ int main(int argc, char** argv)
     else if (name == "no_memory") no_memory();
     else if (name == "no_event") no_event();
     else if (name == "no_record") no_record();
+    else if (name == "small") small();
     else check(false, "unknown scenario");
     return wrong != 0;
 }
