@@ -145,10 +145,22 @@ static hipError_t copy_parallel(HostStage& st, char* dst, const char* src, size_
     return hipError_t(error.load());
 }
 
+// Ordinary host memory is what the runtime does not know.  Into pinned memory
+// its own copy is one transfer at the link's rate (57 GB/s; the threads reach
+// 38 there), and device memory is not the CPU's to write.
+static hipMemoryType memory_type(const void* p)
+{
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type;
+    (void)hipGetLastError();   // (older runtimes call unknown memory an error)
+    return hipMemoryTypeUnregistered;
+}
+
 hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void* src, size_t bytes, hipStream_t s)
 {
     hipDevice_t dev = 0;
-    if (bytes >= SMALL && hipStreamGetDevice(s, &dev) == hipSuccess) {
+    const hipMemoryType to = memory_type(dst);
+    if (bytes >= SMALL && to == hipMemoryTypeUnregistered && hipStreamGetDevice(s, &dev) == hipSuccess) {
         try {
             const CurrentDevice current(dev);
             if (!stage) stage = host_stage(dev);
@@ -162,7 +174,9 @@ hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void
         }
     }
     // one blocking call: 4 KB take 14 us, as an asynchronous copy and a wait 23
-    return hipMemcpyWithStream(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    const hipError_t e = hipMemcpyWithStream(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    if (e != hipSuccess || to == hipMemoryTypeUnregistered || to == hipMemoryTypeHost) return e;
+    return hipStreamSynchronize(s);   // to device memory it may return before the end
 }
 
 }  // namespace lbf

@@ -22,7 +22,8 @@ class HostStage;
 // s (a created stream), and returns when dst is complete.  Works on the
 // stream's device, whichever is current.  `stage` is the caller's handle for
 // that device, taken on the first large copy and kept; any number of threads,
-// each with its own handle, may copy at once.
+// each with its own handle, may copy at once.  dst may also be pinned or device
+// memory.
 hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void* src, size_t bytes, hipStream_t s);
 
 }  // namespace lbf

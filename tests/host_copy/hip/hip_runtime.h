@@ -48,6 +48,11 @@ inline std::atomic<int> records_left{-1};
 // memory that the runtime knows, with its kind
 inline const char *known = nullptr, *known_end = nullptr;
 inline hipMemoryType known_type = hipMemoryTypeUnregistered;
+inline bool knows(const void* p)
+{
+    const char* c = static_cast<const char*>(p);
+    return c >= known && c < known_end;
+}
 
 inline bool spent(std::atomic<int>& left) { return left >= 0 && left-- == 0; }
 inline void drain(FakeStream* s)
@@ -125,13 +130,14 @@ inline hipError_t hipMemcpyWithStream(void* dst, const void* src, size_t n, hipM
 {
     ++fake::plain;
     fake::drain(s);
-    std::memcpy(dst, src, n);
+    // (between device buffers even the blocking call may return before the end)
+    if (fake::knows(dst) && fake::known_type == hipMemoryTypeDevice) s->queued.push_back(FakeCopy{dst, src, n});
+    else std::memcpy(dst, src, n);
     return hipSuccess;
 }
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
 {
-    const char* c = static_cast<const char*>(p);
-    a->type = c >= fake::known && c < fake::known_end ? fake::known_type : hipMemoryTypeUnregistered;
+    a->type = fake::knows(p) ? fake::known_type : hipMemoryTypeUnregistered;
     a->device = 0;
     return hipSuccess;
 }

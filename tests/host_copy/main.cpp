@@ -126,6 +126,26 @@ static void small()
     }
 }
 
+// A destination that the runtime knows: pinned memory, which the device writes by itself,
+// and device memory, which the CPU must not write.
+static void known_memory()
+{
+    FakeStream s;
+    for (hipMemoryType type : {hipMemoryTypeHost, hipMemoryTypeDevice}) {
+        std::shared_ptr<lbf::HostStage> stage;
+        fake::plain = fake::staged = 0;
+        Data d((size_t(20) << 20) + 5);
+        fake::known_type = type;
+        fake::known = d.dst.data();
+        fake::known_end = fake::known + d.dst.size();
+        check(copy(stage, d, &s) == hipSuccess && d.arrived(), "the data have arrived");
+        check(fake::plain == 1 && fake::staged == 0, "by the runtime's own copy");
+        fake::known = fake::known_end = nullptr;
+        Data e((size_t(20) << 20) + 5);
+        check(copy(stage, e, &s) == hipSuccess && e.arrived() && fake::staged > 1, "ordinary memory through the threads");
+    }
+}
+
 int main(int argc, char** argv)
 {
     const std::string name = argc > 1 ? argv[1] : "";
@@ -134,6 +154,7 @@ int main(int argc, char** argv)
     else if (name == "no_event") no_event();
     else if (name == "no_record") no_record();
     else if (name == "small") small();
+    else if (name == "known_memory") known_memory();
     else check(false, "unknown scenario");
     return wrong != 0;
 }

@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize('scenario', ['other_device', 'no_memory', 'no_event', 'no_record', 'small'])
+@pytest.mark.parametrize('scenario', ['other_device', 'no_memory', 'no_event', 'no_record', 'small', 'known_memory'])
 def test_scenario(program, scenario):
     r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
