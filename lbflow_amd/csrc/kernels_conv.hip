@@ -13,8 +13,8 @@
 // channels-last activations and k = tap * Cin + ci, one lane's 8 k are 8
 // consecutive channels of one voxel: a single 16-byte load.
 //
-// Forward, direct kernel (Cin 8 and the 1x1x1 head; the other kernels are
-// described where they stand): a workgroup of 4 waves covers 256 voxels x BN
+// Forward, direct kernel (Cin 8, the 1x1x1 head, and sides below 8 with many
+// samples; the other kernels are described where they stand): a workgroup of 4 waves covers 256 voxels x BN
 // output channels; each wave owns 64 voxels (4 row tiles) x BN.  A is loaded straight from
 // memory into MFMA registers (neighbour gather, 16 B per lane); the weight
 // panel is staged through LDS (128 k per stage, rows padded by 32 B: 72
@@ -665,7 +665,7 @@ conv_fwd_input(ConvGeom g, const __bf16* __restrict__ in, const __bf16* __restri
 // ---------------------------------------------------------------------------
 // forward (and input gradient), 3x3x3 with Cin a multiple of 32, sides below 8
 // (the coarse levels of small volumes): a few dozen voxels against up to 3.5 MB
-// of weights.  One wave per 16 output channels and MT tiles of 16 voxels, in
+// of weights (many samples: the direct kernel).  One wave per 16 output channels and MT tiles of 16 voxels, in
 // the direct kernel's order of k, both operands straight from memory with the
 // loads of FLY k steps in flight: nothing is shared that a barrier would have
 // to wait for.  Bound by the latency of those loads; 256 to 256 channels at
@@ -1348,6 +1348,13 @@ struct ConvLaunch {
     // (256 to 256 channels at 4^3, 8 samples: 38 us, the direct kernel 182), beyond
     // that 4 tiles share a wave's weights (16 samples 49 us, 182; 64: 135, 188)
     static constexpr uint32_t COARSE_VOXELS = 512;
+    // and up to one wave per SIMD.  Each of its waves reads all the weights of its
+    // channels, which at twice as many waves costs more than the direct kernel's
+    // idle CUs: 1024 and 2048 waves, coarse against direct, 64 to 64 channels
+    // 44 / 64 and 75 / 64 us, 256 to 256 131 / 183 and 249 / 208, 384 to 128
+    // 190 / 280 and 367 / 302, 32 to 32 23 / 28 and 31 / 29 (a million voxels of
+    // 256 channels: 30.7 / 9.3 ms).
+    static constexpr uint32_t COARSE_WAVES = 1024;
     // the rows kernel
     static constexpr bool ROWS = HALO && COUT % 32 == 0;
     static constexpr int BN_ROWS = 32;
@@ -1414,29 +1421,32 @@ struct ConvLaunch {
             }
         }
         if constexpr (HALO) {
-            // sides below 8: the coarse kernel, faster than the direct one at every size tried
-            // (2^3 to 4^3, 1 to 64 samples, 32 to 384 channels: 1.4 to 7.8 times)
-            if (g.nvox <= COARSE_VOXELS)
+            // sides below 8: few voxels, the coarse kernel
+            const uint32_t blocks = (g.nvox + 63u) / 64u;
+            if (g.nvox <= COARSE_VOXELS) {
                 hipLaunchKernelGGL((conv_fwd_coarse<CIN, COUT, 1, ACT, BIAS, OUTF32>),
                                    dim3((g.nvox + 15u) / 16u, COUT / 16), dim3(64), 0, s, g, in, w, bias, out);
-            else
-                hipLaunchKernelGGL((conv_fwd_coarse<CIN, COUT, 4, ACT, BIAS, OUTF32>),
-                                   dim3((g.nvox + 63u) / 64u, COUT / 16), dim3(64), 0, s, g, in, w, bias, out);
-        } else {
-            // The input layer with whole 16-byte rows, where a block of 16 x 8 x 8
-            // voxels fits a sample.
-            if constexpr (CIN == 8 && COUT == 32 && TAPS == 27 && !OUTF32 && ACT != ACT_RELU_GATE) {
-                const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out);
-                if (g.log_s >= 4 && at % 16 == 0 && (g.in_stride | g.out_stride) % 8 == 0) {
-                    hipLaunchKernelGGL((conv_fwd_input<ACT, BIAS>), dim3(g.nvox / 1024u), dim3(256), 0, s, g, in, w, bias,
-                                       static_cast<__bf16*>(out));
-                    return;
-                }
+                return;
             }
-            const dim3 grid((g.nvox + 255u) / 256u, (COUT + BN_FWD - 1) / BN_FWD);
-            hipLaunchKernelGGL((conv_fwd<CIN, COUT, TAPS, BN_FWD, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g, in, w,
-                               bias, out);
+            if (blocks <= COARSE_WAVES / (COUT / 16)) {
+                hipLaunchKernelGGL((conv_fwd_coarse<CIN, COUT, 4, ACT, BIAS, OUTF32>), dim3(blocks, COUT / 16), dim3(64),
+                                   0, s, g, in, w, bias, out);
+                return;
+            }
         }
+        // The input layer with whole 16-byte rows, where a block of 16 x 8 x 8
+        // voxels fits a sample.
+        if constexpr (CIN == 8 && COUT == 32 && TAPS == 27 && !OUTF32 && ACT != ACT_RELU_GATE) {
+            const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out);
+            if (g.log_s >= 4 && at % 16 == 0 && (g.in_stride | g.out_stride) % 8 == 0) {
+                hipLaunchKernelGGL((conv_fwd_input<ACT, BIAS>), dim3(g.nvox / 1024u), dim3(256), 0, s, g, in, w, bias,
+                                   static_cast<__bf16*>(out));
+                return;
+            }
+        }
+        const dim3 grid((g.nvox + 255u) / 256u, (COUT + BN_FWD - 1) / BN_FWD);
+        hipLaunchKernelGGL((conv_fwd<CIN, COUT, TAPS, BN_FWD, ACT, BIAS, OUTF32>), grid, dim3(256), 0, s, g, in, w, bias,
+                           out);
     }
     static constexpr int BM_W = COUT >= 64 ? 64 : COUT;
     static constexpr int BN_W = 64;

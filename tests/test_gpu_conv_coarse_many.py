@@ -1,0 +1,64 @@
+"""3x3x3 convolutions at sides below 8 with many samples: the first and last
+sample of a batch on either side of the rule between the kernels equal, bit
+for bit, the same sample alone (the coarse kernel, pinned against the loop
+reference in test_gpu_conv_coarse.py; both add the same products in the same
+order); and many samples cost about what the same voxels cost at side 8."""
+import time
+
+import numpy as np
+import pytest
+
+from lbflow_amd import surrogate as S
+from lbflow_amd.engine import Buffer
+
+pytestmark = pytest.mark.gpu
+
+
+def _conv(cin, cout, side, n, x, w, b, relu=1, f32=0, extra=0):
+    out = Buffer((n * side ** 3, cout + extra), np.float32 if f32 else np.uint16)
+    rc = S.lib().lbf_conv3d_forward(cin, cout, 27, side, n, x.ptr, cin, w.ptr, b.ptr, out.ptr, cout + extra, relu, f32)
+    assert rc == 0, S.lib().lbf_net_error(None)
+    return out
+
+
+# 64 voxels and 16 channels a wave: up to 1024 waves the coarse kernel
+@pytest.mark.parametrize('cin,cout,side,n', [
+    (64, 64, 4, 256), (64, 64, 4, 257), (256, 256, 4, 64), (256, 256, 4, 65), (32, 32, 2, 4097), (96, 32, 1, 32800),
+    (384, 128, 4, 129)])
+@pytest.mark.parametrize('f32', [0, 1])
+def test_sample_alone_equals_in_batch(cin, cout, side, n, f32):
+    rng = np.random.default_rng(cin + 7 * cout + side + n)
+    sv = side ** 3
+    top16 = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    xh = top16(rng.standard_normal((n * sv, cin), dtype=np.float32))
+    w = Buffer((cout, 27 * cin), np.uint16, top16(rng.standard_normal((cout, 27 * cin), dtype=np.float32) * 0.05))
+    b = Buffer((cout,), np.float32, rng.standard_normal(cout).astype(np.float32))
+    whole = _conv(cin, cout, side, n, Buffer(xh.shape, np.uint16, xh), w, b, f32=f32, extra=8).numpy()
+    for s in (0, n - 1):
+        part = xh[s * sv:(s + 1) * sv]
+        alone = _conv(cin, cout, side, 1, Buffer(part.shape, np.uint16, part), w, b, f32=f32, extra=8).numpy()
+        assert np.array_equal(alone, whole[s * sv:(s + 1) * sv])
+
+
+@pytest.mark.parametrize('cin,cout', [(256, 256), (64, 64)])
+def test_many_samples_cost(cin, cout):
+    """131072 voxels at side 4 within 2.5 times the same at side 8: 1.2 and 1.4
+    times measured with 256 channels and 64; 4.7 and 4.1 with a wave per 64
+    voxels and 16 channels, which reads all weights for every 64 voxels."""
+    nv = 131072
+    x, w, b = Buffer((nv, cin), np.uint16), Buffer((cout, 27 * cin), np.uint16), Buffer((cout,), np.float32)
+    out = Buffer((nv, cout), np.uint16)
+
+    def best(side):
+        t = []
+        for _ in range(8):
+            t0 = time.perf_counter()
+            rc = S.lib().lbf_conv3d_forward(cin, cout, 27, side, nv // side ** 3, x.ptr, cin, w.ptr, b.ptr, out.ptr,
+                                            cout, 1, 0)
+            t.append(time.perf_counter() - t0)
+            assert rc == 0
+        return min(t[2:])
+
+    a, c = best(4), best(8)
+    print('side 4', a * 1e6, 'side 8', c * 1e6, flush=True)
+    assert a < 2.5 * c
