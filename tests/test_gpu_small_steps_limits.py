@@ -1,19 +1,21 @@
 """FP64 steps several to a launch, where their rules end: two-phase work orders
 whose padded entries just fill or just miss the limit (the count is asserted,
 so that each case runs the kernel it is there for), per-site relaxation times
-in D3Q19, more steps than one launch holds.  advance(n) equals n single steps bit
-for bit."""
+in D3Q19, more steps than one launch holds; and single-phase lattices with
+Zou-He boundaries.  advance(n) equals n single steps bit for bit, and with
+Zou-He boundaries also the CPU oracle."""
 import numpy as np
 import pytest
 
 from lbflow_amd import cases as CS
+from tests import cases as TC
 
 pytestmark = pytest.mark.gpu
 
 
-def _engine(spec, solids):
+def _engine(spec, solids, dense=False):
     from lbflow_amd.engine import FP64, Engine
-    return Engine(CS.lattice(spec), CS.geometry(spec), FP64, solids).init()
+    return Engine(CS.lattice(spec), CS.geometry(spec), FP64, solids, dense).init()
 
 
 def _items(geom, solids):
@@ -55,3 +57,24 @@ def test_colour_limits(shape, phi, eq, solids, harmonic, several):
             b.step(0)
         assert a.t == b.t and a.status()[0] == b.status()[0] == 0
         assert np.array_equal(a.populations().view(np.uint64), b.populations().view(np.uint64))
+
+
+@pytest.mark.parametrize('spec', TC.zouhe_cases(nx=12, ny=7, nz=6), ids=lambda s: s['name'])
+def test_zouhe_advance(spec):
+    case, geom = CS.lattice(spec), CS.geometry(spec)
+    assert geom.size <= (1024 if case['D'] == 2 else 512)
+    from oracle.pyoracle import Oracle
+    a, single, orc = _engine(spec, True), _engine(spec, True), Oracle(case, geom).init()
+    f, fsingle = _engine(spec, False, True), _engine(spec, False, True)
+    for n in (1, 2, 7, 150):
+        a.advance(n)
+        f.advance(n)
+        for _ in range(n):
+            single.step(0)
+            fsingle.step(0)
+        orc.step(n)
+        pa, po = a.populations(), orc.populations()
+        assert np.array_equal(pa.view(np.uint64), single.populations().view(np.uint64))
+        assert np.array_equal(pa.view(np.uint64), po.view(np.uint64))
+        assert np.array_equal(f.populations().view(np.uint64), fsingle.populations().view(np.uint64))
+    assert a.status()[0] == 0 and f.status()[0] == 0
