@@ -1358,13 +1358,6 @@ struct ConvLaunch {
     // the rows kernel
     static constexpr bool ROWS = HALO && COUT % 32 == 0;
     static constexpr int BN_ROWS = 32;
-    // For 32 output channels its workgroups are twice the halo kernel's, and where
-    // all of those run at once (up to one per CU) they end no sooner: halo
-    // against rows, 32 to 32 channels gated 16 x 16^3 10.1 / 11.1 us, 64 to 32 in
-    // two splits 6 x 16^3 16.9 / 18.4, 96 to 32 6 x 16^3 21.6 / 22.9.  The next step up
-    // (half as many more voxels) the rows kernel wins: 23.6 / 20.4, 41 / 31, and
-    // 96 channels from 192 workgroups on 36 / 33.
-    static constexpr uint32_t ROWS_ABOVE = COUT != 32 ? 0 : CIN > 64 ? 128 : 256;
 
     template <int ACT, bool BIAS, bool OUTF32>
     static void fwd(const ConvGeom& g, const __bf16* in, const __bf16* w, const float* bias, void* out, hipStream_t s)
@@ -1402,7 +1395,7 @@ struct ConvLaunch {
                     const bool gated = ACT == ACT_RELU_GATE;
                     const uintptr_t at = uintptr_t(in) | uintptr_t(w) | uintptr_t(out) | (gated ? uintptr_t(g.gate) : 0);
                     const uint32_t strides = g.in_stride | g.out_stride | (gated ? g.gate_stride : 0u);
-                    rows = !few && wgs * ks > ROWS_ABOVE && g.log_s >= 4 && sample_bytes < (uint64_t(1) << 32) && at % 16 == 0 && strides % 8 == 0;
+                    rows = !few && g.log_s >= 4 && sample_bytes < (uint64_t(1) << 32) && at % 16 == 0 && strides % 8 == 0;
                     if (rows) {
                         const dim3 grid(g.nvox / 512u * (COUT / BN_ROWS), ks);
                         __bf16* o = static_cast<__bf16*>(out);
