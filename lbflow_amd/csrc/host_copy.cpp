@@ -173,10 +173,16 @@ hipError_t copy_to_host(std::shared_ptr<HostStage>& stage, void* dst, const void
             // out of host memory or threads: the plain copy below
         }
     }
-    // one blocking call: 4 KB take 14 us, as an asynchronous copy and a wait 23
-    const hipError_t e = hipMemcpyWithStream(dst, src, bytes, hipMemcpyDeviceToHost, s);
-    if (e != hipSuccess || to == hipMemoryTypeUnregistered || to == hipMemoryTypeHost) return e;
-    return hipStreamSynchronize(s);   // to device memory it may return before the end
+    if (to != hipMemoryTypeUnregistered && to != hipMemoryTypeHost) {
+        // device memory: even the blocking call may return before the end
+        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipStreamSynchronize(s);
+    }
+    // The blocking call after the stream's work is the quickest for small results: fields of
+    // 320 sites 27 us, 35 by hipMemcpyWithStream and 44 by an asynchronous copy and a wait
+    // (200 steps, a report and the fields 508, 527 and 525).
+    const hipError_t e = hipStreamSynchronize(s);
+    return e != hipSuccess ? e : hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
 }
 
 }  // namespace lbf

@@ -126,13 +126,10 @@ inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpy
     s->queued.push_back(FakeCopy{dst, src, n});
     return hipSuccess;
 }
-inline hipError_t hipMemcpyWithStream(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t s)
+inline hipError_t hipMemcpy(void* dst, const void* src, size_t n, hipMemcpyKind)
 {
-    ++fake::plain;
-    fake::drain(s);
-    // (between device buffers even the blocking call may return before the end)
-    if (fake::knows(dst) && fake::known_type == hipMemoryTypeDevice) s->queued.push_back(FakeCopy{dst, src, n});
-    else std::memcpy(dst, src, n);
+    ++fake::plain;   // (of the null stream: nothing of another stream is waited for)
+    std::memcpy(dst, src, n);
     return hipSuccess;
 }
 inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p)
