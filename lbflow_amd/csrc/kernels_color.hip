@@ -27,8 +27,11 @@
 // FP64, reference operation order (built with -ffp-contract=off); zero
 // lattice coefficients are skipped exactly as in kernels_scsp.hip.
 //
-// Bound: FP64 issue and, on lattices of a few waves per SIMD, the step's own
-// chain of cold loads and cold code (220 registers, two waves per SIMD).
+// Bound: on large lattices FP64 issue; on lattices of about a wave per SIMD the
+// life of one wave (48^3: VALU issue 17 % of the cycles, half of a wave's time
+// goes by waiting to issue, a third for memory).  The D3Q19 MRT step holds 240
+// registers (any site kind 224, CSF 218), two waves per SIMD, and spills 83-118
+// SGPRs to VGPR lanes.
 // Waves hold either fluid or solid sites (setup.h build_items), the operators
 // come through scalar loads (operator_f64.h; through vector loads they were 480
 // round trips), directions are divided by the gradient's norm once per opposite

@@ -209,9 +209,14 @@ __device__ __forceinline__ void scsp_site_f64(const ScspParams& p, const DevLabe
 // ---------------------------------------------------------------------------
 // FP64, reference operation order.
 //
-// Bound, MRT: half by HBM, half by FP64 issue (1444 of about 2300 FP64
-// instructions are the two operator products, add_operator).  One site per
-// lane, 151 registers, three waves per SIMD.  Measured per step on dense
+// Bound, MRT, 125 x 112 x 120: the loads that 2.5 waves per SIMD keep in flight (HBM
+// 542 MB a step, 4.0 TB/s, 65 % of the copy kernel's rate), with VALU issue at 69 %
+// of the cycles behind them (1444 of a fluid wave's about 2300 FP64 instructions are
+// the two operator products, add_operator).  Taking most of that issue away, by
+// packing a workgroup's fluid sites into consecutive lanes through LDS, left
+// 131 us of 132 (and made 13.4 at 48^3 15.2).  At 48^3, one round of 1728 waves, it is the
+// life of one wave.  One site per lane, 151-165 registers (sparse 137), three
+// waves per SIMD.  Measured per step on dense
 // sphere packs of porosity 0.2-0.24, before and after the operators moved from
 // LDS to scalar loads and the solid sites joined the fluid sites' loads and
 // stores: 125 x 112 x 120 229 -> 132 us (3.9 TB/s), 48^3 18.7 -> 13.4 us, an
