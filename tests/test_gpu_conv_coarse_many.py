@@ -42,8 +42,8 @@ def test_sample_alone_equals_in_batch(cin, cout, side, n, f32):
 
 @pytest.mark.parametrize('cin,cout', [(256, 256), (64, 64)])
 def test_many_samples_cost(cin, cout):
-    """131072 voxels at side 4 within 2.5 times the same at side 8: 1.2 and 1.4
-    times measured with 256 channels and 64; 4.7 and 4.1 with a wave per 64
+    """131072 voxels at side 4 within 2.5 times the same at side 8: 1.4 and 1.3
+    times measured with 256 channels and 64; 4.7 and 3.7 with a wave per 64
     voxels and 16 channels, which reads all weights for every 64 voxels."""
     nv = 131072
     x, w, b = Buffer((nv, cin), np.uint16), Buffer((cout, 27 * cin), np.uint16), Buffer((cout,), np.float32)
